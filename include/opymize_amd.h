@@ -538,7 +538,10 @@ int opy_conv3x3_fwd_bf16(const float* x, float* y, const void* wt, const float* 
  * same results at half the traffic), 0 for float32 */
 int opy_conv3x3_fwd_io(const void* x, void* y, const void* wt, const float* bias, int N, int H, int W, int act,
                        int x_bf16, int y_bf16, int grid, void* stream);
-/* per-block partials (grid x (9*32*32 + 32) floats) of dW[tap][co][ci] and dbias[co] */
+/* backward-data through the ReLU of the layer below: y = conv(g, W) where mask > 0, else 0 (mask: that layer's
+ * output, of y's shape; wt from opy_conv3x3_prep_weights with flip = 1); g 16-byte aligned */
+int opy_conv3x3_bwd_data(const float* g, float* y, const void* wt, const float* mask, int N, int H, int W, int grid,
+                         void* stream);
 /* The warm start's first layer straight from packed images (no counterpart): input channel 0 =
  * f - 0.5, channel 1 = loglam[n], channels 2..31 = 0 for image n at f + n*stride (H*W floats);
  * output NHWC BF16, 32 channels, ReLU. */
@@ -549,10 +552,16 @@ int opy_conv3x3_first(const float* f, int64_t stride, const float* loglam, void*
  * f / x_out + n*stride and y_out + 2n*stride; x 16-byte and y_out 8-byte aligned. */
 int opy_conv3x3_last(const void* x, const float* f, int64_t stride, float* x_out, float* y_out, const void* wt,
                      const float* bias, int N, int H, int W, int grid, void* stream);
+/* per-block partials (grid x (9*32*32 + 32) floats) of dW[tap][co][ci] and dbias[co] */
 int opy_conv3x3_wgrad_bf16(const float* x, const float* g, float* partials, int N, int H, int W, int grid,
                            void* stream);
-/* out[i] = sum_b partials[b*len + i] in block order */
+/* out[i] = sum_b partials[b*len + i], in an order fixed by nb */
 int opy_sum_partials_f32(const float* partials, int nb, int len, float* out, void* stream);
+/* a layer's weight and bias gradients from nb partials of opy_conv3x3_wgrad_bf16: out[tap][ci][co], then dbias[co] */
+int opy_conv3x3_grad_reduce(const float* partials, int nb, float* out, void* stream);
+/* opy_conv3x3_prep_weights of `layers` layers, whose FP32 weights start `per` floats apart, in both directions:
+ * wf, wb (layers x 9*32*32 bf16) */
+int opy_conv3x3_prep_all(const float* params, int64_t per, int layers, void* wf, void* wb, void* stream);
 /* master weights W[tap][ci][co] (float) -> bf16 [tap][co][ci]; flip=1 gives the backward-data weights */
 int opy_conv3x3_prep_weights(const float* w, void* out, int flip, void* stream);
 /* g *= (y > 0) */

@@ -33,8 +33,11 @@ def _bind():
         "opy_conv3x3_fwd_io": [P, P, P, P, I, I, I, I, I, I, I, P],
         "opy_conv3x3_first": [P, L, P, P, P, P, I, I, I, I, P],
         "opy_conv3x3_last": [P, P, L, P, P, P, P, I, I, I, I, P],
+        "opy_conv3x3_bwd_data": [P, P, P, P, I, I, I, I, P],
         "opy_conv3x3_wgrad_bf16": [P, P, P, I, I, I, I, P],
         "opy_sum_partials_f32": [P, I, I, P, P],
+        "opy_conv3x3_grad_reduce": [P, I, P, P],
+        "opy_conv3x3_prep_all": [P, L, I, P, P, P],
         "opy_conv3x3_prep_weights": [P, P, I, P],
         "opy_relu_bwd_f32": [P, P, L, P],
         "opy_adam_f32": [P, P, P, P, I, D, D, D, D, I, P],
@@ -79,9 +82,16 @@ class ConvNet(object):
         self.v = torch.zeros_like(self.params)
         self.step = 0
         self.n_in, self.n_out = n_in, n_out
-        self._wf = [torch.empty(9 * CH * CH, dtype=torch.bfloat16, device="cuda") for _ in range(layers)]
-        self._wb = [torch.empty(9 * CH * CH, dtype=torch.bfloat16, device="cuda") for _ in range(layers)]
-        self.grid = 8 * torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+        # BF16 weights of all layers, forward and backward-data, and each layer's part
+        self._wf_all = torch.empty(layers * 9 * CH * CH, dtype=torch.bfloat16, device="cuda")
+        self._wb_all = torch.empty_like(self._wf_all)
+        self._wf = list(self._wf_all.split(9 * CH * CH))
+        self._wb = list(self._wb_all.split(9 * CH * CH))
+        cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+        self.grid = 8 * cus
+        # blocks of the weight-gradient kernel: two per CU keep its loads in flight, and each
+        # block's partial gradient is written and read once more
+        self.wgrad_blocks = 2 * cus
         self._dirty = True
         self._ibufs = {}  # inference buffers by input shape: two BF16 activations and the float32 output
 
@@ -95,10 +105,8 @@ class ConvNet(object):
     def _prep(self):
         if not self._dirty:
             return
-        s = _hip.stream()
-        for l in range(self.layers):
-            _call("opy_conv3x3_prep_weights", _hip.ptr(self.W(l)), _hip.ptr(self._wf[l]), 0, s)
-            _call("opy_conv3x3_prep_weights", _hip.ptr(self.W(l)), _hip.ptr(self._wb[l]), 1, s)
+        _call("opy_conv3x3_prep_all", _hip.ptr(self.params), self.per, self.layers, _hip.ptr(self._wf_all),
+              _hip.ptr(self._wb_all), _hip.stream())
         self._dirty = False
 
     def state_dict(self):
@@ -191,23 +199,20 @@ class ConvNet(object):
         """Gradients of all parameters into self.grads given dL/d(output)."""
         N, H, W, _ = gout.shape
         s = _hip.stream()
-        nb = min(self.grid, N * ((H + 15) // 16) * ((W + 15) // 16))
+        nb = min(self.wgrad_blocks, N * ((H + 7) // 8) * ((W + 31) // 32))
         part = torch.empty(nb * self.per, dtype=torch.float32, device="cuda")
+        bufs = [torch.empty_like(gout) for _ in range(min(2, self.layers - 1))]
         g = gout
         for l in range(self.layers - 1, -1, -1):
-            if l < self.layers - 1:
-                _call("opy_relu_bwd_f32", _hip.ptr(g), _hip.ptr(acts[l + 1]), g.numel(), s)
             _call("opy_conv3x3_wgrad_bf16", _hip.ptr(acts[l]), _hip.ptr(g), _hip.ptr(part), N, H, W, nb, s)
-            gl = self.grads[l * self.per:(l + 1) * self.per]
-            # partials hold dW as [tap][co][ci]; reorder to the master [tap][ci][co] below
-            tmp = torch.empty(self.per, dtype=torch.float32, device="cuda")
-            _call("opy_sum_partials_f32", _hip.ptr(part), nb, self.per, _hip.ptr(tmp), s)
-            gl[:9 * CH * CH].copy_(tmp[:9 * CH * CH].view(9, CH, CH).transpose(1, 2).reshape(-1))
-            gl[9 * CH * CH:].copy_(tmp[9 * CH * CH:])
+            # fold the partials, from [tap][co][ci] to the master's [tap][ci][co]
+            _call("opy_conv3x3_grad_reduce", _hip.ptr(part), nb,
+                  _hip.ptr(self.grads[l * self.per:(l + 1) * self.per]), s)
             if l > 0:
-                gn = torch.empty_like(g)
-                _call("opy_conv3x3_fwd_bf16", _hip.ptr(g), _hip.ptr(gn), _hip.ptr(self._wb[l]), None, N, H, W, 0,
-                      self.grid, s)
+                # dL/d(output of layer l - 1) through its ReLU: zero where that output is not positive
+                gn = bufs[l % 2]
+                _call("opy_conv3x3_bwd_data", _hip.ptr(g), _hip.ptr(gn), _hip.ptr(self._wb[l]), _hip.ptr(acts[l]),
+                      N, H, W, self.grid, s)
                 g = gn
         return self.grads
 
