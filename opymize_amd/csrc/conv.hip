@@ -12,14 +12,15 @@
 //   D (16 x 16): col l%16, rows 4*(l/16) .. 4*(l/16)+3
 #include "opy_common.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace opy {
 namespace {
 
 constexpr int kCh = 32;              // channels
-constexpr int kTW = 32, kTH = 16;    // output tile of the forward kernels
-constexpr int kHW = kTW + 2, kHH = kTH + 2;
+constexpr int kTW = 32;              // output tile width of the forward kernels
+constexpr int kHW = kTW + 2;
 constexpr int kPixStride = kCh + 8;  // bf16 elements per LDS pixel (padding against bank conflicts)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -55,32 +56,35 @@ struct ConvIO {
 // half the traffic).
 //
 // An implicit GEMM per tap, D (16 out channels x 16 pixels of a row) += W (16 x
-// 32) * x (32 x 16).  A block of four wavefronts computes 32 x 16 output pixels;
+// 32) * x (32 x 16).  A block of four wavefronts computes 32 x kTH output pixels;
 // its input with the one-pixel halo sits in LDS as BF16, and the next tile's
 // input is on its way into registers meanwhile.  What the layers move bounds
 // them (64-128 B per pixel against 18.4 kflop), so everything else is kept off
 // the path:
 // - The weights of all taps stay in registers (72 of them), and an input row's
 //   three column shifts are read from LDS once for the three output rows that
-//   use them: 36 LDS reads per 144 matrix instructions of a wavefront's tile.
-//   With the weights in LDS and a read per tap they were 54 for 72, and LDS was
-//   busier than the matrix cores.
+//   use them: with 16 rows 36 LDS reads per 144 matrix instructions of a
+//   wavefront's tile.  With the weights in LDS and a read per tap they were 54
+//   for 72, and LDS was busier than the matrix cores.
 // - The rows of W are permuted so that lane (pixel l%16, l/16) ends up with the
 //   8 consecutive output channels 8*(l/16)..: the results leave straight from
 //   registers, 16 or 32 bytes per lane and whole pixels per quarter wavefront,
 //   where they used to be staged through LDS between two barriers.
 // - Consecutive tiles go to the blocks of one XCD, whose L2 then serves the
 //   halos.
+// 8 x 1024^2, BF16 in and out: 295 -> 203 us a layer (5.3 TB/s); 32 x 128^2,
+// FP32: 44 -> 25 us (5.3 TB/s).
 // Accumulation per output runs over dy, dx and the 32 input channels in this
 // order in every instantiation, so all of them give the same bits.
-template <int MODE, typename TX, typename TY, bool kMask>
+template <int MODE, typename TX, typename TY, bool kMask, int kTH>
 __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ x, TY* __restrict__ y,
                                                          const __bf16* __restrict__ wt,
                                                          const float* __restrict__ bias,
                                                          const float* __restrict__ mask, int N, int H, int W, int act,
                                                          ConvIO io) {
   constexpr int NJ = MODE == kLast ? 1 : 2;  // blocks of 16 output channels
-  constexpr int NHP = kHW * kHH;             // pixels of a halo tile
+  constexpr int RW = kTH / 4;                // output rows of a wavefront
+  constexpr int NHP = kHW * (kTH + 2);       // pixels of a halo tile
   constexpr int NV = MODE == kFirst ? NHP : NHP * (kCh / 8);  // staged vectors (kFirst: image values)
   constexpr int NPF = (NV + 255) / 256;
   __shared__ __align__(16) __bf16 xs[MODE == kFirst ? 2 * NHP : NHP * kPixStride];
@@ -118,7 +122,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
   // the next tile's input: image values, BF16 vectors, or FP32 vectors (rounded on the way to LDS)
   float pf[MODE == kFirst ? NPF : 1];
   bf16x8 pv[MODE != kFirst && sizeof(TX) == 2 ? NPF : 1];
-  f32x4 pw[MODE != kFirst && sizeof(TX) == 4 ? NPF : 1][2];
+  f32x4 pa[MODE != kFirst && sizeof(TX) == 4 ? NPF : 1], pb[MODE != kFirst && sizeof(TX) == 4 ? NPF : 1];
   auto prefetch = [&](int t) {
     int n, h0, w0;
     origin(t, n, h0, w0);
@@ -136,11 +140,13 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
           pv[i] = bf16x8{};
           if (in) pv[i] = *reinterpret_cast<const bf16x8*>(s);
         } else {
-          pw[i][0] = pw[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+          f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = a;
           if (in) {
-            pw[i][0] = *reinterpret_cast<const f32x4*>(s);
-            pw[i][1] = *reinterpret_cast<const f32x4*>(s + 4);
+            a = *reinterpret_cast<const f32x4*>(s);
+            b = *reinterpret_cast<const f32x4*>(s + 4);
           }
+          pa[i] = a;
+          pb[i] = b;
         }
       }
     }
@@ -165,12 +171,8 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
         const int e = tid + 256 * i;
         if (e >= NV) continue;
         bf16x8 v;
-        if constexpr (sizeof(TX) == 2) {
-          v = pv[i];
-        } else {
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[k] = to_bf16(pw[i][k >> 2][k & 3]);
-        }
+        if constexpr (sizeof(TX) == 2) v = pv[i];
+        else v = __builtin_convertvector(__builtin_shufflevector(pa[i], pb[i], 0, 1, 2, 3, 4, 5, 6, 7), bf16x8);
         *reinterpret_cast<bf16x8*>(xs + (e >> 2) * kPixStride + 8 * (e & 3)) = v;
       }
     }
@@ -181,22 +183,31 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
     __syncthreads();  // every wavefront is done with the previous tile
     to_lds(t);
     __syncthreads();
-    if (t + G < ntiles) prefetch(t + G);
     int n, h0, w0;
     origin(t, n, h0, w0);
+    float fc[MODE == kLast ? 2 * RW : 1];
+    if constexpr (MODE == kLast) {
+      // the pixels' own image values, on their way before the next tile's input
+#pragma unroll
+      for (int k = 0; k < 2 * RW; ++k) {
+        const int h = h0 + wave * RW + k % RW, w = w0 + (k / RW) * 16 + li;
+        fc[k] = (lk == 0 && h < H && w < W) ? io.f[(int64_t)n * io.stride + (int64_t)h * W + w] : 0.f;
+      }
+    }
+    if (t + G < ntiles) prefetch(t + G);
 #pragma unroll
     for (int cb = 0; cb < kTW / 16; ++cb) {
-      // wavefront `wave` has the output rows 4*wave .. 4*wave+3 of the tile
-      f32x4 acc[4][NJ];
+      // wavefront `wave` has the output rows RW*wave .. RW*wave + RW-1 of the tile
+      f32x4 acc[RW][NJ];
 #pragma unroll
-      for (int m = 0; m < 4; ++m)
+      for (int m = 0; m < RW; ++m)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 6; ++i)
+      for (int i = 0; i < RW + 2; ++i)
 #pragma unroll
         for (int dx = 0; dx < 3; ++dx) {
-          const int p = (wave * 4 + i) * kHW + cb * 16 + li + dx;
+          const int p = (wave * RW + i) * kHW + cb * 16 + li + dx;
           bf16x8 b;
           if constexpr (MODE == kFirst) {
             u32x4 v = {0u, 0u, 0u, 0u};
@@ -207,7 +218,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
             b = *reinterpret_cast<const bf16x8*>(xs + p * kPixStride + 8 * lk);
           }
 #pragma unroll
-          for (int m = 0; m < 4; ++m) {
+          for (int m = 0; m < RW; ++m) {
             const int dy = i - m;
             if (dy < 0 || dy > 2) continue;
 #pragma unroll
@@ -217,8 +228,8 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
         }
       const int w = w0 + cb * 16 + li;
 #pragma unroll
-      for (int m = 0; m < 4; ++m) {
-        const int h = h0 + wave * 4 + m;
+      for (int m = 0; m < RW; ++m) {
+        const int h = h0 + wave * RW + m;
         if (h >= H || w >= W) continue;
         float v[4 * NJ];
 #pragma unroll
@@ -229,7 +240,7 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
         if constexpr (MODE == kLast) {
           if (lk == 0) {
             const int64_t q = (int64_t)n * io.stride + (int64_t)h * W + w;
-            io.xo[q] = ((io.f[q] - 0.5f) + 0.5f) + v[0];
+            io.xo[q] = ((fc[cb * RW + m] - 0.5f) + 0.5f) + v[0];
             *reinterpret_cast<float2*>(io.yo + 2 * q) = make_float2(v[1], v[2]);
           }
         } else {
@@ -256,14 +267,21 @@ __global__ void __launch_bounds__(256, 2) conv3x3_kernel(const TX* __restrict__ 
   }
 }
 
-// `grid` blocks at most, and no more than there are tiles or than keep every CU busy with resident
-// blocks (each block reads the weights once): rounded down to the 8 XCDs
-constexpr int kConvBlocks = 512;  // two per CU
-inline int conv_grid(int N, int H, int W, int grid) {
-  const int64_t tiles = (int64_t)N * ((H + kTH - 1) / kTH) * ((W + kTW - 1) / kTW);
-  int64_t g = grid < tiles ? grid : tiles;
-  if (g > kConvBlocks) g = kConvBlocks;
-  return (int)(g > 8 ? g - g % 8 : g);
+// Two blocks per CU hold the weights and the next tile's input in registers; each block walks
+// several tiles. Output rows per tile, measured on a 32 x 128^2 batch (FP32 in and out) and on
+// 8 x 1024^2 (BF16): FP32 input 8 rows 25 us a layer (5.3 TB/s), 16 rows 28 us (the next tile takes
+// 80 registers), without loading ahead 28-30 us; BF16 input 16 rows 203 us a layer (5.3 TB/s),
+// 8 rows 212 us, without loading ahead 245 us.
+template <int MODE, typename TX, typename TY, bool kMask>
+void launch_conv(const TX* x, TY* y, const void* wt, const float* bias, const float* mask, int N, int H, int W,
+                 int act, const ConvIO& io, int grid, hipStream_t st) {
+  constexpr int TH = sizeof(TX) == 4 ? 8 : 16;
+  constexpr int kMost = 512;
+  const int64_t tiles = (int64_t)N * ((H + TH - 1) / TH) * ((W + kTW - 1) / kTW);
+  int64_t g = std::min<int64_t>(std::min(grid, kMost), tiles);
+  if (g > 8) g -= g % 8;  // whole rounds of the 8 XCDs
+  hipLaunchKernelGGL((conv3x3_kernel<MODE, TX, TY, kMask, TH>), dim3((unsigned)g), dim3(256), 0, st, x, y,
+                     static_cast<const __bf16*>(wt), bias, mask, N, H, W, act, io);
 }
 
 // ---- backward-weights ----------------------------------------------------------
@@ -503,8 +521,7 @@ OPY_API int opy_conv3x3_fwd_bf16(const float* x, float* y, const void* wt, const
   if (!x || !y || !wt || N < 1 || H < 1 || W < 1 || grid < 1) return fail(kInvalid, "conv3x3_fwd: bad arguments");
   if (x == y) return fail(kInvalid, "conv3x3_fwd: in-place convolution is not supported");
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(kInvalid, "conv3x3_fwd: input must be 16-byte aligned");
-  hipLaunchKernelGGL((conv3x3_kernel<kPlain, float, float, false>), dim3(conv_grid(N, H, W, grid)), dim3(256), 0,
-                     as_stream(s), x, y, static_cast<const __bf16*>(wt), bias, nullptr, N, H, W, act, ConvIO{});
+  launch_conv<kPlain, float, float, false>(x, y, wt, bias, nullptr, N, H, W, act, ConvIO{}, grid, as_stream(s));
   return check_launch("conv3x3_fwd");
 }
 OPY_API int opy_conv3x3_bwd_data(const float* g, float* y, const void* wt, const float* mask, int N, int H, int W,
@@ -514,8 +531,7 @@ OPY_API int opy_conv3x3_bwd_data(const float* g, float* y, const void* wt, const
   if (g == y || mask == y) return fail(kInvalid, "conv3x3_bwd_data: the output must not alias an input");
   if ((reinterpret_cast<uintptr_t>(g) & 15) != 0)
     return fail(kInvalid, "conv3x3_bwd_data: input must be 16-byte aligned");
-  hipLaunchKernelGGL((conv3x3_kernel<kPlain, float, float, true>), dim3(conv_grid(N, H, W, grid)), dim3(256), 0,
-                     as_stream(s), g, y, static_cast<const __bf16*>(wt), nullptr, mask, N, H, W, 0, ConvIO{});
+  launch_conv<kPlain, float, float, true>(g, y, wt, nullptr, mask, N, H, W, 0, ConvIO{}, grid, as_stream(s));
   return check_launch("conv3x3_bwd_data");
 }
 OPY_API int opy_conv3x3_fwd_io(const void* x, void* y, const void* wt, const float* bias, int N, int H, int W,
@@ -526,24 +542,19 @@ OPY_API int opy_conv3x3_fwd_io(const void* x, void* y, const void* wt, const flo
   if (y_bf16 && (reinterpret_cast<uintptr_t>(y) & 15) != 0)
     return fail(kInvalid, "conv3x3_fwd_io: BF16 output must be 16-byte aligned");
   const __bf16* w = static_cast<const __bf16*>(wt);
-  const dim3 gr(conv_grid(N, H, W, grid));
   hipStream_t st = as_stream(s);
   const __bf16* xh = static_cast<const __bf16*>(x);
   const float* xf = static_cast<const float*>(x);
   __bf16* yh = static_cast<__bf16*>(y);
   float* yf = static_cast<float*>(y);
   if (x_bf16 && y_bf16)
-    hipLaunchKernelGGL((conv3x3_kernel<kPlain, __bf16, __bf16, false>), gr, dim3(256), 0, st, xh, yh, w, bias, nullptr,
-                       N, H, W, act, ConvIO{});
+    launch_conv<kPlain, __bf16, __bf16, false>(xh, yh, w, bias, nullptr, N, H, W, act, ConvIO{}, grid, st);
   else if (x_bf16)
-    hipLaunchKernelGGL((conv3x3_kernel<kPlain, __bf16, float, false>), gr, dim3(256), 0, st, xh, yf, w, bias, nullptr,
-                       N, H, W, act, ConvIO{});
+    launch_conv<kPlain, __bf16, float, false>(xh, yf, w, bias, nullptr, N, H, W, act, ConvIO{}, grid, st);
   else if (y_bf16)
-    hipLaunchKernelGGL((conv3x3_kernel<kPlain, float, __bf16, false>), gr, dim3(256), 0, st, xf, yh, w, bias, nullptr,
-                       N, H, W, act, ConvIO{});
+    launch_conv<kPlain, float, __bf16, false>(xf, yh, w, bias, nullptr, N, H, W, act, ConvIO{}, grid, st);
   else
-    hipLaunchKernelGGL((conv3x3_kernel<kPlain, float, float, false>), gr, dim3(256), 0, st, xf, yf, w, bias, nullptr,
-                       N, H, W, act, ConvIO{});
+    launch_conv<kPlain, float, float, false>(xf, yf, w, bias, nullptr, N, H, W, act, ConvIO{}, grid, st);
   return check_launch("conv3x3_fwd_io");
 }
 
@@ -553,9 +564,7 @@ OPY_API int opy_conv3x3_first(const float* f, int64_t stride, const float* logla
     return fail(kInvalid, "conv3x3_first: bad arguments");
   if ((reinterpret_cast<uintptr_t>(y) & 15) != 0) return fail(kInvalid, "conv3x3_first: output must be 16-byte aligned");
   ConvIO io{f, stride, loglam, nullptr, nullptr};
-  hipLaunchKernelGGL((conv3x3_kernel<kFirst, __bf16, __bf16, false>), dim3(conv_grid(N, H, W, grid)), dim3(256), 0,
-                     as_stream(s), nullptr, static_cast<__bf16*>(y), static_cast<const __bf16*>(wt), bias, nullptr, N,
-                     H, W, 1, io);
+  launch_conv<kFirst, __bf16, __bf16, false>(static_cast<const __bf16*>(nullptr), static_cast<__bf16*>(y), wt, bias, nullptr, N, H, W, 1, io, grid, as_stream(s));
   return check_launch("conv3x3_first");
 }
 OPY_API int opy_conv3x3_last(const void* x, const float* f, int64_t stride, float* xo, float* yo, const void* wt,
@@ -565,9 +574,7 @@ OPY_API int opy_conv3x3_last(const void* x, const float* f, int64_t stride, floa
   if ((reinterpret_cast<uintptr_t>(x) & 15) != 0) return fail(kInvalid, "conv3x3_last: input must be 16-byte aligned");
   if ((reinterpret_cast<uintptr_t>(yo) & 7) != 0) return fail(kInvalid, "conv3x3_last: yo must be 8-byte aligned");
   ConvIO io{f, stride, nullptr, xo, yo};
-  hipLaunchKernelGGL((conv3x3_kernel<kLast, __bf16, __bf16, false>), dim3(conv_grid(N, H, W, grid)), dim3(256), 0,
-                     as_stream(s), static_cast<const __bf16*>(x), nullptr, static_cast<const __bf16*>(wt), bias,
-                     nullptr, N, H, W, 0, io);
+  launch_conv<kLast, __bf16, __bf16, false>(static_cast<const __bf16*>(x), static_cast<__bf16*>(nullptr), wt, bias, nullptr, N, H, W, 0, io, grid, as_stream(s));
   return check_launch("conv3x3_last");
 }
 

@@ -278,3 +278,64 @@ def test_warm_start_at_full_size_matches_oracle_windows(gpu):
             y_ref = y_ref * np.minimum(1.0, 1.0 / np.maximum(nrm, 1e-300))  # |y| <= tvw = 1
             rel_close(X[r0:r0 + h, c0:c0 + w], x_ref)
             rel_close(Y[r0:r0 + h, c0:c0 + w], y_ref)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 8, 32), (1, 9, 33), (3, 17, 65), (1, 40, 31)])
+def test_conv_kernels_at_tile_edges(gpu, shape):
+    """The forward kernel's tiles are 32 x 8 (float32 input) and 32 x 16
+    (BF16), the weight gradient's 32 x 8: sizes at, below and just past them.
+    Forward in float32 and BF16, backward-data through the ReLU mask, and the
+    weight gradients with their reduction, against the oracle (2e-3 of the
+    output scale, as above; the bias gradient is an FP32 sum of float32
+    values, 1e-5)."""
+    from opymize_amd.warmstart.cnn import ConvNet, _call
+    from opymize_amd import _hip
+    N, H, W = shape
+    rng = np.random.default_rng(N + H + W)
+    net = ConvNet(layers=1, n_in=32, n_out=32, seed=7)
+    net._prep()
+    Wm = net.W(0).cpu().numpy().reshape(9, 32, 32)
+    x = rng.standard_normal((N, H, W, 32)).astype(np.float32)
+    g = rng.standard_normal((N, H, W, 32)).astype(np.float32)
+    xd, gd = torch.as_tensor(x).cuda(), torch.as_tensor(g).cuda()
+    s = _hip.stream()
+    ref = cnn.conv_fwd(x, Wm, np.zeros(32, dtype=np.float32), relu=False)
+    for dt in (torch.float32, torch.bfloat16):
+        xi, y = xd.to(dt), torch.full_like(xd, 7.0)
+        _call("opy_conv3x3_fwd_io", _hip.ptr(xi), _hip.ptr(y), _hip.ptr(net._wf[0]), None, N, H, W, 0,
+              int(dt == torch.bfloat16), 0, net.grid, s)
+        rel_close(y.cpu().numpy(), ref)
+    dx = torch.full_like(gd, 7.0)
+    _call("opy_conv3x3_bwd_data", _hip.ptr(gd), _hip.ptr(dx), _hip.ptr(net._wb[0]), _hip.ptr(xd), N, H, W, net.grid, s)
+    out = dx.cpu().numpy()
+    rel_close(out, cnn.conv_bwd_data(g, Wm) * (x > 0))
+    assert np.all(out[x <= 0] == 0.0)
+    nb = min(net.wgrad_blocks, N * ((H + 7) // 8) * ((W + 31) // 32))
+    part = torch.empty(nb * net.per, dtype=torch.float32, device="cuda")
+    tot = torch.empty(net.per, dtype=torch.float32, device="cuda")
+    _call("opy_conv3x3_wgrad_bf16", _hip.ptr(xd), _hip.ptr(gd), _hip.ptr(part), N, H, W, nb, s)
+    _call("opy_conv3x3_grad_reduce", _hip.ptr(part), nb, _hip.ptr(tot), s)
+    t = tot.cpu().numpy()
+    dW_ref, db_ref = cnn.conv_bwd_weights(x, g)
+    rel_close(t[:9 * 1024].reshape(9, 32, 32), dW_ref)
+    rel_close(t[9 * 1024:], db_ref, tol=1e-5)
+
+
+@pytest.mark.parametrize("nb", [1, 7, 16, 129])
+def test_partial_sums_over_segments(gpu, nb):
+    """16 segments of the partials per column: fewer partials than segments,
+    a multiple, a remainder; the transposed form gives the same values."""
+    from opymize_amd.warmstart.cnn import _bind, _call
+    from opymize_amd import _hip
+    _bind()
+    per = 9 * 32 * 32 + 32
+    part = torch.randn(nb * per, device="cuda", generator=torch.Generator("cuda").manual_seed(nb))
+    a, b = torch.empty(per, device="cuda"), torch.empty(per, device="cuda")
+    _call("opy_sum_partials_f32", _hip.ptr(part), nb, per, _hip.ptr(a), _hip.stream())
+    _call("opy_conv3x3_grad_reduce", _hip.ptr(part), nb, _hip.ptr(b), _hip.stream())
+    p = part.view(nb, per).double()
+    # nb float32 additions of values of size 1: nb ulps of the sum of magnitudes
+    tol = nb * 1.2e-7 * p.abs().sum(0)
+    assert bool(((a.double() - p.sum(0)).abs() <= tol).all())
+    w = a[:9 * 1024].view(9, 32, 32).transpose(1, 2).reshape(-1)
+    assert torch.equal(b[:9 * 1024], w) and torch.equal(b[9 * 1024:], a[9 * 1024:])
