@@ -431,6 +431,22 @@ int opy_tv_stream_f64(const double* x_in, double* x_out, const double* y_in, dou
  * strips carry no halo beyond the image edge: 1 for W <= 64, else ceil((W - 64) / sw) + 1. */
 int opy_tv_stream_units(const opy_tv_inst_t* insts, const int32_t* active_inst, const int32_t* nact,
                         int32_t* unit_off, int k, int rows, void* stream);
+/* The same k in 2..8 iterations for one-channel FP32 batches, bit for bit, with two image columns per lane:
+ * units of 128-2k columns by `rows` rows (strips(W) = the smaller of ceil(W / sw), sw = 128 - 2k, and of the
+ * layout whose first and last strips carry no halo beyond the image edge: 1 for W <= 128, else
+ * ceil((W - 128) / sw) + 1).  The launch runs the iterations it0 .. it0+k-1 of the n whose coefficients
+ * opy_tv_wide_steps wrote to `table`; `grid` > 0 wavefronts (blocks of 64) walk the units.
+ *   opy_tv_wide_steps: the coefficients of the next n iterations of every running instance's schedule (SCALAR or
+ *     ACCEL steps) to table (B x n x 8 floats, 32-byte aligned) and, with ACCEL, its state advanced by n;
+ *   opy_tv_wide_units: the exclusive prefix of the running instances' units of these strips (wide_off), and of
+ *     opy_tv_stream_units' (stream_off), B+1 entries each. */
+int opy_tv_wide_f32(const float* x_in, float* x_out, const float* y_in, float* y_out, const float* f,
+                    const opy_tv_inst_t* insts, const float* table, int n, int it0, const int32_t* active_inst,
+                    const int32_t* unit_off, const int32_t* nact, int k, int rows, int grid, void* stream);
+int opy_tv_wide_steps(const opy_tv_inst_t* insts, opy_adapt_state_t* steps, const opy_tv_check_t* checks, int B,
+                      const opy_tv_cfg_t* cfg, int n, float* table, void* stream);
+int opy_tv_wide_units(const opy_tv_inst_t* insts, const int32_t* active_inst, const int32_t* nact, int k,
+                      int32_t* stream_off, int stream_rows, int32_t* wide_off, int wide_rows, void* stream);
 /* adaptive step rule per running instance from the residual partials (reference pdhg.py:155-183) */
 int opy_tv_adapt(const opy_tv_inst_t* insts, opy_adapt_state_t* steps, const opy_tv_check_t* checks,
                  const double* partials, int B, int C, const opy_adapt_params_t* params, void* stream);

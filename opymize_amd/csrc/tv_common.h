@@ -498,6 +498,30 @@ __device__ inline double readlane(double v, int l) {
                           __builtin_amdgcn_readlane(__double2loint(v), l));
 }
 
+// ---- strips of the streaming kernel (tv_stream.hip; counted in tv_wide.hip too) ----
+// Strips of an instance W columns wide.  Plainly, strip s holds the exact
+// columns [s sw, (s + 1) sw) (sw = 64 - 2K) on lanes K .. 63 - K, lane 0 on
+// column s sw - K: ceil(W / sw) strips.  Extended, when that takes fewer
+// strips: the first strip needs no halo beyond the left image edge, whose
+// boundary the stencils' masks close, so lane 0 sits on column 0 and lanes
+// 0 .. 63 - K are exact; the last (the one whose lanes reach column W - 1)
+// needs none beyond the right edge, so its exact lanes run to 63; lane 0 of
+// strip s sits on column s sw, and n strips cover 64 + (n - 1) sw columns.
+// The plain layout keeps the strip edges where they are better aligned for
+// the row loads and stores (3-7% faster at equal strip counts), which wins
+// where HBM bounds the launch: the extended one is taken only from K = 6
+// (sw <= 52), where instruction issue does (1024 columns at K = 8: 21
+// strips instead of 22, 3.5% faster; at K = 2: 17 instead of 18, but 3.5%
+// slower).
+__host__ __device__ inline int stream_strips_plain(int W, int sw) { return (W + sw - 1) / sw; }
+__host__ __device__ inline int stream_strips_ext(int W, int sw) { return W <= 64 ? 1 : (W - 64 + sw - 1) / sw + 1; }
+__host__ __device__ inline bool stream_extended(int W, int sw) {
+  return sw <= 52 && stream_strips_ext(W, sw) < stream_strips_plain(W, sw);
+}
+__host__ __device__ inline int stream_strips(int W, int sw) {
+  return stream_extended(W, sw) ? stream_strips_ext(W, sw) : stream_strips_plain(W, sw);
+}
+
 // ---- host wrappers ---------------------------------------------------------
 #define KF(...) reinterpret_cast<const void*>(&__VA_ARGS__)
 

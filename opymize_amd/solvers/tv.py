@@ -62,6 +62,8 @@ CHECK_DOUBLES = ctypes.sizeof(TVCheck) // 8
 RESTART_DOUBLES = ctypes.sizeof(TVRestart) // 8
 STATE_DOUBLES = _hip.ADAPT_STATE_DOUBLES
 STREAM_MIN_UNITS = 4096
+WIDE_COLS = 128   # columns of a strip of the two-column streaming kernel
+WIDE_TABLE = 64   # iterations whose step coefficients it takes from one table
 assert ctypes.sizeof(TVInst) == 48 and ctypes.sizeof(TVCfg) == 64 and ctypes.sizeof(TVCheck) == 72
 assert ctypes.sizeof(TVRestart) == 24
 
@@ -85,6 +87,11 @@ _PLAIN = {
     "opy_tv_compact": [ctypes.c_void_p] * 2 + [ctypes.c_int] + [ctypes.c_void_p] * 4 + [ctypes.c_int,
                                                                                       ctypes.c_void_p],
     "opy_tv_stream_units": [ctypes.c_void_p] * 4 + [ctypes.c_int, ctypes.c_int, ctypes.c_void_p],
+    "opy_tv_wide_f32": [ctypes.c_void_p] * 7 + [ctypes.c_int] * 2 + [ctypes.c_void_p] * 3 + [ctypes.c_int] * 3 +
+                       [ctypes.c_void_p],
+    "opy_tv_wide_steps": [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_int] + [ctypes.c_void_p] * 2,
+    "opy_tv_wide_units": [ctypes.c_void_p] * 3 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
+                                                  ctypes.c_int, ctypes.c_void_p],
 }
 _bound = False
 
@@ -119,6 +126,36 @@ def _stream_strips(W, sw):
     return min(plain, ext) if sw <= 52 else plain
 
 
+def _wide_strips(W, sw):
+    """Strips of the two-column streaming kernel (the kernel's wide_strips)."""
+    return np.minimum(-(-W // sw), np.where(W <= WIDE_COLS, 1, -(-(W - WIDE_COLS) // sw) + 1))
+
+
+# rows per unit that the two-column kernel may take (wide_rows)
+WIDE_ROWS = (8, 10, 12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 52, 57, 64, 69, 74, 80, 86, 94, 103, 114, 128,
+             147, 171, 205, 256, 342, 512)
+
+
+def wide_rows(H, strips, k, simds):
+    """Rows per unit of the two-column streaming kernel for running instances
+    of H rows and `strips` strips each.
+
+    A unit of R rows walks R + 2k of them, so few tall units are cheap; but a
+    SIMD runs two units at once, in 1.54 of the time units that one alone
+    takes 0.95 of, and those left over when the others have ended leave most
+    of the chip idle.  (Microseconds per row step, measured at 8 iterations
+    per launch on 32 and 128 images of 1024^2 with 48 to 256 rows: within 10%
+    of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)"""
+    best, rows = None, WIDE_ROWS[-1]
+    for R in WIDE_ROWS:
+        u = float(np.sum(strips * -(-H // R))) / simds
+        rounds, rest = divmod(u, 2.0)
+        cost = (R + 2 * k) * (1.54 * rounds + (0.0 if rest < 0.01 else 0.95 if rest <= 1.0 else 1.54))
+        if best is None or cost < best:
+            best, rows = cost, R
+    return rows
+
+
 def tile_height(tw, rpt):
     return (256 // tw) * rpt
 
@@ -143,11 +180,13 @@ class TVBatch(object):
     multi_kernel: how K > 1 iterations per launch are split over the GPU:
             "stream" (one wavefront per strip of 64 - 2K columns by
             stream_rows rows, the K iterations pipelined down the rows), "tile"
-            (LDS-staged tiles, K <= 4), or "auto": stream while the running
-            instances give at least stream_min_units units (decided at each
-            check), else tiles with min(K, 4) iterations per launch, and
-            tiles for preconditioned steps; every choice gives the iterates
-            of single launches bit for bit
+            (LDS-staged tiles, K <= 4), or "auto": one-channel FP32 batches
+            stream strips of 128 - 2K columns, two per lane, whose rows per
+            unit follow from the running instances (wide_rows); others stream
+            while the running instances give at least stream_min_units units
+            (decided at each check), else take tiles with min(K, 4) iterations
+            per launch; preconditioned steps take tiles.  Every choice gives
+            the iterates of single launches bit for bit
     stream_rows: rows per unit of the streaming kernel
     """
 
@@ -195,8 +234,14 @@ class TVBatch(object):
             raise ValueError("multi_kernel must be 'auto', 'stream' or 'tile'")
         self.multi_kernel = multi_kernel
         self.unit_off = torch.zeros(self.B + 1, dtype=torch.int32, device="cuda")
+        self.wide_off = torch.zeros(self.B + 1, dtype=torch.int32, device="cuda")
         self.stream_rows = 128
         self.total_units, self.sgrid = 0, 0
+        self._H = np.array([H for (H, W) in self.shapes], dtype=np.int64)
+        self._W = np.array([W for (H, W) in self.shapes], dtype=np.int64)
+        self._simds = 4 * torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+        self.wrows, self.wgrid, self._wide_sized = 128, 8, None
+        self._wide_table = None
         # "auto" streams while the running instances give at least this many
         # units (about four wavefronts per SIMD), else takes the tile kernel
         self.stream_min_units = STREAM_MIN_UNITS
@@ -232,8 +277,11 @@ class TVBatch(object):
         if self.multi < 2:
             self.total_units = 0
             return
+        self._wide_sized = None
+        self._size_wide(np.arange(self.B))
         sw, rows = 64 - 2 * self.multi, self.stream_rows
-        self.total_units = sum(_stream_strips(W, sw) * (-(-H // rows)) for (H, W) in self.shapes)
+        self._strips = np.array([_stream_strips(W, sw) for (H, W) in self.shapes], dtype=np.int64)
+        self.total_units = int(np.sum(self._strips * -(-self._H // rows)))
         if self._grid_override is None:
             self.sgrid = self._stream_grid(self.total_units)
         else:
@@ -244,8 +292,26 @@ class TVBatch(object):
     def _stream_units(self):
         if self.multi > 1:
             P = _hip.ptr
-            self._call("opy_tv_stream_units", P(self.insts), P(self.active_inst), P(self.nact), P(self.unit_off),
-                       self.multi, self.stream_rows, _hip.stream())
+            self._call("opy_tv_wide_units", P(self.insts), P(self.active_inst), P(self.nact), self.multi,
+                       P(self.unit_off), self.stream_rows, P(self.wide_off), self.wrows, _hip.stream())
+
+    def _size_wide(self, running):
+        """Rows per unit and blocks of the two-column streaming kernel for the
+        running instances; True if the rows changed.  Both follow the running
+        set in steps of a sixteenth of the batch, so that a solve needs few
+        distinct launch shapes (one captured graph each); blocks past the
+        running units return at once."""
+        strips = _wide_strips(self._W, WIDE_COLS - 2 * self.multi)
+        work = strips * self._H
+        share = -(-16 * int(work[running].sum()) // int(work.sum())) if len(running) else 0
+        if share == self._wide_sized or share == 0:
+            return False
+        self._wide_sized = share
+        was = self.wrows
+        self.wrows = wide_rows(self._H[running], strips[running], self.multi, self._simds)
+        units = int(np.sum(strips[running] * -(-self._H[running] // self.wrows)))
+        self.wgrid = -(-max(units, 1) // 8) * 8
+        return self.wrows != was
 
     def _stream_grid(self, units):
         """Blocks (4 wavefronts, one unit each) for `units` running units,
@@ -273,6 +339,11 @@ class TVBatch(object):
             return False
         return self.multi_kernel == "stream" or self._stream_now
 
+    def _use_wide(self, cfg):
+        """Whether the next K-iteration launches run the two-column streaming kernel."""
+        return (self.multi_kernel == "auto" and self.multi > 1 and self.C == 1 and self.dtype == torch.float32
+                and cfg.steps != STEP_MODES["precond"] and self._stream_fits())
+
     def _stream_fits(self):
         """Every instance's y block (2 C values per pixel) is below 4 GiB, the
         reach of the streaming kernel's 32-bit offsets."""
@@ -282,7 +353,7 @@ class TVBatch(object):
     def _launch_k(self, cfg):
         """Iterations per K-iteration launch: multi, or at most 4 on the tile
         kernel (the same iterates, grouped differently)."""
-        return self.multi if self._use_stream(cfg) else min(self.multi, 4)
+        return self.multi if self._use_wide(cfg) or self._use_stream(cfg) else min(self.multi, 4)
 
     def set_tile(self, tw, rpt):
         if self.passes == 1:
@@ -311,9 +382,11 @@ class TVBatch(object):
         self.insts = torch.as_tensor(raw).cuda()
         self.part_res = torch.zeros(4 * t0, dtype=torch.float64, device="cuda")
         self.part_gap = torch.zeros(6 * t0, dtype=torch.float64, device="cuda")
-        self.active_inst = torch.zeros(self.B, dtype=torch.int32, device="cuda")
-        self.act_off = torch.zeros(self.B + 1, dtype=torch.int32, device="cuda")
-        self.nact = torch.zeros(1, dtype=torch.int32, device="cuda")
+        # the running instances: their number, indices and tile prefix, read back in one copy
+        self._running = torch.zeros(2 * self.B + 2, dtype=torch.int32, device="cuda")
+        self.nact = self._running[:1]
+        self.active_inst = self._running[1:self.B + 1]
+        self.act_off = self._running[self.B + 1:]
         self.iter_counter = torch.zeros(1, dtype=torch.int64, device="cuda")
         # by default every launch gets one block per tile of the running
         # instances, rounded up to a bucket (see _launch_grid), which keeps the
@@ -340,14 +413,17 @@ class TVBatch(object):
     def refresh_grid(self):
         """Read the running tile count (one device read) and size the
         following launches to it; returns the number of running instances."""
-        nrun = int(self.nact.item())
-        tiles = int(self.act_off[nrun].item()) if nrun > 0 else 0
-        self.grid = self._launch_grid(tiles)
+        run = self._running.cpu().numpy()
+        nrun = int(run[0])
+        running = run[1:1 + nrun]
+        self.grid = self._launch_grid(int(run[self.B + 1 + nrun]))
         if self.multi > 1:
-            units = int(self.unit_off[nrun].item()) if nrun > 0 else 0
+            units = int(np.sum(self._strips[running] * -(-self._H[running] // self.stream_rows)))
             if self._grid_override is None:
                 self.sgrid = self._stream_grid(units)
             self._stream_now = units >= self.stream_min_units
+            if self._size_wide(running):
+                self._stream_units()
         return nrun
 
     def _cfg(self, steps):
@@ -472,9 +548,32 @@ class TVBatch(object):
         if cfg.steps == STEP_MODES["accel"]:
             self._call("opy_tv_accel_n", P(self.insts), P(self.state), P(self.checks), self.B, int(k), s)
 
+    def _wide_iterations(self, n, cfg, k):
+        """The first n - n % k of n iterations on the two-column streaming
+        kernel, k per launch; returns n % k."""
+        P = _hip.ptr
+        s = _hip.stream()
+        if self._wide_table is None:
+            self._wide_table = torch.zeros(self.B * WIDE_TABLE * 8, dtype=torch.float32, device="cuda")
+        while n >= k:
+            m = min(n, WIDE_TABLE)
+            m -= m % k
+            self._call("opy_tv_wide_steps", P(self.insts), P(self.state), P(self.checks), self.B, ctypes.byref(cfg), m,
+                       P(self._wide_table), s)
+            for it0 in range(0, m, k):
+                p = self.cur
+                self._call("opy_tv_wide_f32", P(self.x[p]), P(self.x[1 - p]), P(self.y[p]), P(self.y[1 - p]),
+                           P(self.f), P(self.insts), P(self._wide_table), m, it0, P(self.active_inst),
+                           P(self.wide_off), P(self.nact), int(k), self.wrows, self.wgrid, s)
+                self.cur ^= 1
+            n -= m
+        return n
+
     def _iterations(self, n, cfg, adapt, params):
         """n iterations starting from buffer self.cur (updates self.cur)."""
         k = self._launch_k(cfg) if not adapt else 1
+        if k > 1 and n >= k and self._use_wide(cfg):
+            n = self._wide_iterations(n, cfg, k)
         while k > 1 and n >= k:
             self._multi_launch(self.cur, cfg, k)
             self.cur ^= 1
@@ -498,7 +597,7 @@ class TVBatch(object):
         block of a solve runs eagerly, which loads its kernels before any
         capture; a new key is captured (that records without running) and
         then replayed."""
-        key = (self.grid, self.sgrid, self._stream_now, self.cur)
+        key = (self.grid, self.sgrid, self._stream_now, self.wrows, self.wgrid, self.cur)
         if key in cache:
             g, end = cache[key]
             g.replay()

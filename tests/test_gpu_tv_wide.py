@@ -1,0 +1,97 @@
+"""The two-column streaming kernel (opy_tv_wide, TVBatch(multi_kernel="auto")
+on one-channel FP32 batches): strips of 128 - 2K columns, two per lane.  Its
+iterates are those of K single launches bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_tv_batch import rects
+
+pytestmark = pytest.mark.gpu
+
+# widths at and around one strip (128), two strips of the extended layout
+# (128 + 128 - 2K) and of the plain one, odd ones, one column; heights of one
+# row, below and above the units' rows and the 2K steps before the first store
+SHAPES = [(130, 200), (1, 100), (97, 1), (5, 128), (40, 129), (17, 113), (23, 241), (64, 2), (150, 127), (30, 371),
+          (200, 256)]
+
+
+def _run(multi, kernel, steps, rows, monkeypatch, shapes=SHAPES, iters=24):
+    from opymize_amd.solvers import tv
+    monkeypatch.setattr(tv, "WIDE_ROWS", (rows,))
+    imgs = [rects(H, W, 3 + i) for i, (H, W) in enumerate(shapes)]
+    lams = [1.0 + 1.7 * i for i in range(len(shapes))]
+    data = ["l1" if i % 3 == 1 else "l2" for i in range(len(shapes))]
+    bat = tv.TVBatch(imgs, lams, data, tvw=[1.0 + 0.1 * i for i in range(len(shapes))], tile=(64, 4), multi=multi,
+                     multi_kernel=kernel)
+    res = bat.solve(steps=steps, step_bound=0.124, max_iters=2 * iters, block_iters=iters, tol=1e-30)
+    if multi > 1:
+        assert bat._use_wide(bat._cfg(steps)) == (kernel == "auto") and bat.wrows == rows
+    return bat.solution(), [r["gap"] for r in res]
+
+
+@pytest.mark.parametrize("steps", ["accel", "const"])
+@pytest.mark.parametrize("multi,rows", [(2, 8), (3, 40), (4, 8), (5, 256), (6, 32), (7, 8), (8, 8), (8, 40), (8, 256)])
+def test_wide_equals_single_launches(gpu, monkeypatch, multi, rows, steps):
+    """Two blocks of a whole number of launches and a remainder of single
+    iterations (25 = 3 * 8 + 1), TV-L1 and TV-L2, uneven TV weights."""
+    (xs, ys), gaps = _run(multi, "auto", steps, rows, monkeypatch, iters=25)
+    (x1, y1), gaps1 = _run(1, "auto", steps, rows, monkeypatch, iters=25)
+    for a, b in zip(xs + ys, x1 + y1):
+        np.testing.assert_array_equal(a, b)
+    assert gaps == gaps1
+
+
+def test_wide_units_follow_the_running_instances(gpu):
+    """The device's unit prefixes against a host recount, after some
+    instances stopped; rows chosen for the whole and the reduced set."""
+    import torch
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 9 + i) for i, (H, W) in enumerate(SHAPES)]
+    bat = tv.TVBatch(imgs, 3.0, "l2", multi=8)
+    bat.solve(steps="accel", step_bound=0.124, max_iters=8, block_iters=8, tol=1e-30)
+    ck = bat.checks.view(torch.int32).reshape(bat.B, -1)
+    for b in (0, 4, 10):
+        ck[b, 16] = 1  # status field of opy_tv_check_t: certified
+    bat._compact(0)
+    nrun = bat.refresh_grid()
+    active = bat.active_inst.cpu().numpy()[:nrun]
+    assert nrun == bat.B - 3 and not {0, 4, 10} & set(active.tolist())
+    for off, strips, rows in ((bat.wide_off, tv._wide_strips(bat._W, 112), bat.wrows),
+                              (bat.unit_off, bat._strips, bat.stream_rows)):
+        counts = (strips * -(-bat._H // rows))[active]
+        np.testing.assert_array_equal(off.cpu().numpy()[:nrun + 1], np.concatenate([[0], np.cumsum(counts)]))
+
+
+def test_wide_graph_replays_equal_eager(gpu):
+    """Captured blocks (the step table among them) replayed many times against
+    eager launches, on a batch that certifies instance by instance."""
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
+    out = []
+    for g in (True, False):
+        bat = tv.TVBatch(imgs, [2.0, 9.0, 15.0, 19.0], "l2", multi=8)
+        res = bat.solve(steps="accel", step_bound=0.124, step_factor=4.0, max_iters=4800, block_iters=48, tol=1e-5,
+                        use_graph=g)
+        out.append(([(r["iter"], r["gap"], r["status"]) for r in res], bat.solution()))
+    assert out[0][0] == out[1][0] and all(s == 1 for _, _, s in out[0][0])
+    for a, b in zip(out[0][1][0] + out[0][1][1], out[1][1][0] + out[1][1][1]):
+        np.testing.assert_array_equal(a, b)
+
+
+def test_wide_entry_points_refuse_bad_arguments():
+    """Host checks before any launch."""
+    import ctypes
+    from opymize_amd import _hip
+    from opymize_amd.solvers import tv
+    tv._bind()
+    lib = _hip.load()
+    assert lib.opy_tv_wide_f32(*([None] * 7), 8, 0, None, None, None, 9, 8, 8, None) == 1
+    assert b"k = 9" in lib.opy_last_error()
+    q = ctypes.c_void_p(64)
+    args = [q, ctypes.c_void_p(128), q, ctypes.c_void_p(128), q, q, q]
+    assert lib.opy_tv_wide_f32(*args, 8, 1, q, q, q, 8, 8, 8, None) == 1  # iterations 1..9 of 8
+    assert b"outside the table" in lib.opy_last_error()
+    c = tv.TVCfg()
+    c.C, c.tw, c.rpt, c.steps, c.h0, c.h1 = 1, 64, 4, tv.STEP_MODES["precond"], 1.0, 1.0
+    assert lib.opy_tv_wide_steps(q, q, q, 1, ctypes.byref(c), 8, q, None) == 1
+    assert b"preconditioned" in lib.opy_last_error()
