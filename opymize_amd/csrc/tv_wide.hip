@@ -7,7 +7,7 @@ namespace opy {
 namespace {
 
 // Work unit: one wavefront per (strip, chunk) of an instance, as in
-// tv_stream_kernel: the wavefront walks down R + 2K rows, loads each row of x,
+// tv_stream_kernel; the chunks of an instance share its rows evenly.  The wavefront walks down R + 2K rows, loads each row of x,
 // f and y once and runs the K iterations as a pipeline skewed by one row per
 // level.  Lane l holds the columns 2l and 2l + 1 of a strip of 128 columns, of
 // which 128 - 2K are exact.
@@ -67,23 +67,39 @@ __host__ __device__ inline int wide_strips(int W, int sw) {
 
 // iteration i (< n) of every running instance's step schedule: its coefficients
 // to tab[b * n + i], and the instance's state n iterations on (the FP64
-// operations of tv_accel_kernel and fold_step)
+// operations of tv_accel_kernel and fold_step).  One wavefront per instance: the
+// schedule is a serial chain of square roots and divisions, the coefficients
+// that hang off it are formed by one lane per iteration.
 __global__ void __launch_bounds__(64) tv_steps_kernel(const opy_tv_inst_t* __restrict__ insts,
                                                       opy_adapt_state_t* __restrict__ st,
-                                                      const opy_tv_check_t* __restrict__ chk, int B, Cfg cfg, int n,
+                                                      const opy_tv_check_t* __restrict__ chk, Cfg cfg, int n,
                                                       WideStep* __restrict__ tab) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B || chk[b].status != 0) return;
+  const int b = blockIdx.x;
+  if (chk[b].status != 0) return;
   const opy_tv_inst_t I = insts[b];
   double tau = st[b].tau, sigma = st[b].sigma;
-  for (int i = 0; i < n; ++i) {
-    const double th = accel_theta(cfg.steps, I, tau);
-    const FoldedStep<float, 1> s = fold_step<float, 1>(tau, sigma / th, th, I, cfg);
-    tab[(int64_t)b * n + i] = {s.a, s.b, s.theta, 1.0f + s.theta, s.p[0][0], s.p[1][0], s.q[0][0], s.q[1][0]};
-    tau *= th;
-    sigma /= th;
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    // every lane walks the chain and keeps its own iteration's values
+    double mt = 0.0, ms = 0.0, mth = 1.0;
+    const int m = min(64, n - i0);
+    for (int i = 0; i < m; ++i) {
+      const double th = accel_theta(cfg.steps, I, tau);
+      const double so = sigma / th;
+      if ((int)threadIdx.x == i) {
+        mt = tau;
+        ms = so;
+        mth = th;
+      }
+      tau *= th;
+      sigma = so;
+    }
+    if ((int)threadIdx.x < m) {
+      const FoldedStep<float, 1> s = fold_step<float, 1>(mt, ms, mth, I, cfg);
+      tab[(int64_t)b * n + i0 + threadIdx.x] = {s.a,       s.b,       s.theta,   1.0f + s.theta,
+                                                s.p[0][0], s.p[1][0], s.q[0][0], s.q[1][0]};
+    }
   }
-  if (cfg.steps == OPY_TV_STEPS_ACCEL) {
+  if (cfg.steps == OPY_TV_STEPS_ACCEL && threadIdx.x == 0) {
     st[b].tau = tau;
     st[b].sigma = sigma;
   }
@@ -110,17 +126,18 @@ __global__ void __launch_bounds__(64, K >= 7 ? 2 : (K >= 5 ? 3 : 4)) tv_wide_ker
                                                       const WideStep* __restrict__ tab, int tab_n, int it0,
                                                       const int32_t* __restrict__ active_inst,
                                                       const int32_t* __restrict__ unit_off,
-                                                      const int32_t* __restrict__ nact_p, int R) {
+                                                      const int32_t* __restrict__ nact_p, int rows) {
   constexpr int SW = kWideCols - 2 * K;
   const int nact = *nact_p;
   if (nact <= 0) return;
   const int total = unit_off[nact];
-  const int NSTEP = R + 2 * K;
   const int lane = threadIdx.x;
   for (int u = xcd_block(); u < total; u += gridDim.x) {
-    const TileRef tr = locate(u, active_inst, unit_off, nact, insts, SW, R);
+    const TileRef tr = locate(u, active_inst, unit_off, nact, insts, SW, rows);
     const opy_tv_inst_t I = insts[tr.b];
     const int H = I.H, W = I.W;
+    const int nc = (H + rows - 1) / rows, R = (H + nc - 1) / nc;  // chunks, and their rows (at most `rows`)
+    const int NSTEP = R + 2 * K;
     const int ns = wide_strips(W, SW), ty = tr.j / ns;
     const bool ext = ns < (W + SW - 1) / SW;
     const int r0 = ty * R - K;  // image row of pipeline row 0
@@ -265,8 +282,11 @@ __global__ void __launch_bounds__(64, K >= 7 ? 2 : (K >= 5 ? 3 : 4)) tv_wide_ker
           OPY_J v[j] = __builtin_fmaf(v[j], s.p0, xcur[j]);
           OPY_J v[j] = __builtin_fmaf(y1[j], s.p1, v[j]);
           if constexpr (L1) {
+            // soft_rest, the clamp as one median (a NaN stays one in the difference)
+            float cl[2];
             OPY_J v[j] = v[j] - F[i][j];
-            OPY_J v[j] = soft_rest(v[j], s.b);
+            OPY_J cl[j] = __builtin_amdgcn_fmed3f(v[j], -s.b, s.b);
+            OPY_J v[j] = v[j] - cl[j];
             OPY_J xnew[j] = F[i][j] + v[j];
           } else {
             OPY_J v[j] = __builtin_fmaf(s.b, F[i][j], v[j]);
@@ -421,8 +441,8 @@ OPY_API int opy_tv_wide_steps(const opy_tv_inst_t* insts, opy_adapt_state_t* st,
   if (!insts || !st || !chk || !table || B < 1 || n < 1) return fail(kInvalid, "tv_wide_steps: bad arguments");
   if ((reinterpret_cast<uintptr_t>(table) & 31) != 0)
     return fail(kInvalid, "tv_wide_steps: the table must be 32-byte aligned");
-  hipLaunchKernelGGL(tv_steps_kernel, dim3((B + 63) / 64), dim3(64), 0, as_stream(s), insts, st, chk, B, make_cfg(cfg),
-                     n, reinterpret_cast<WideStep*>(table));
+  hipLaunchKernelGGL(tv_steps_kernel, dim3(B), dim3(64), 0, as_stream(s), insts, st, chk, make_cfg(cfg), n,
+                     reinterpret_cast<WideStep*>(table));
   return check_launch("tv_wide_steps");
 }
 

@@ -140,7 +140,8 @@ def wide_rows(H, strips, k, simds):
     """Rows per unit of the two-column streaming kernel for running instances
     of H rows and `strips` strips each.
 
-    A unit of R rows walks R + 2k of them, so few tall units are cheap; but a
+    An instance of H rows is cut into ceil(H / R) chunks of even height, and a
+    unit of r rows walks r + 2k of them, so few tall units are cheap; but a
     SIMD runs two units at once, in 1.54 of the time units that one alone
     takes 0.95 of, and those left over when the others have ended leave most
     of the chip idle.  (Microseconds per row step, measured at 8 iterations
@@ -148,9 +149,12 @@ def wide_rows(H, strips, k, simds):
     of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)"""
     best, rows = None, WIDE_ROWS[-1]
     for R in WIDE_ROWS:
-        u = float(np.sum(strips * -(-H // R))) / simds
-        rounds, rest = divmod(u, 2.0)
-        cost = (R + 2 * k) * (1.54 * rounds + (0.0 if rest < 0.01 else 0.95 if rest <= 1.0 else 1.54))
+        chunks = -(-H // R)
+        units = strips * chunks
+        n = float(np.sum(units))
+        steps = float(np.sum(units * (-(-H // chunks) + 2 * k))) / n  # of a unit, on average
+        rounds, rest = divmod(n / simds, 2.0)
+        cost = steps * (1.54 * rounds + (0.0 if rest < 0.01 else 0.95 if rest <= 1.0 else 1.54))
         if best is None or cost < best:
             best, rows = cost, R
     return rows
