@@ -527,6 +527,15 @@ int opy_lift_dual_f32(const float* Ub, const float* rb, float* p, float* z, cons
 int opy_lift_dual_f64(const double* Ub, const double* rb, double* p, double* z, const double* f,
                       const opy_lift_inst_t* insts, const int32_t* active_inst, const int32_t* act_off,
                       const int32_t* nact, int kmax, int grid, void* stream);
+/* both passes in one: reads U, r, p, z and f, writes r in place and U, p, z to their other buffers; the iterates of
+ * a primal and a dual pass.  kmax <= 32 (FP64: 16). */
+int opy_lift_iter_f32(const float* U_in, float* U_out, float* r, const float* p_in, float* p_out, const float* z_in,
+                      float* z_out, const float* f, const opy_lift_inst_t* insts, const int32_t* active_inst,
+                      const int32_t* act_off, const int32_t* nact, int kmax, int grid, void* stream);
+int opy_lift_iter_f64(const double* U_in, double* U_out, double* r, const double* p_in, double* p_out,
+                      const double* z_in, double* z_out, const double* f, const opy_lift_inst_t* insts,
+                      const int32_t* active_inst, const int32_t* act_off, const int32_t* nact, int kmax, int grid,
+                      void* stream);
 /* FP64 gap partials, 8 per tile (reference pdhg.py:23-44 for this model) */
 int opy_lift_gap_f32(const float* U, const float* r, const float* p, const float* z, const float* f,
                      const opy_lift_inst_t* insts, const int32_t* active_inst, const int32_t* act_off,

@@ -34,6 +34,7 @@ P, I, L, D = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_double
 _SIGS = {
     "opy_lift_primal": [P, P, P, P, P, P, P, P, P, P, I, I, P],
     "opy_lift_dual": [P, P, P, P, P, P, P, P, P, I, I, P],
+    "opy_lift_iter": [P, P, P, P, P, P, P, P, P, P, P, P, I, I, P],
     "opy_lift_gap": [P, P, P, P, P, P, P, P, P, I, P, I, P],
 }
 _PLAIN = {
@@ -128,10 +129,16 @@ class LiftBatch(object):
         self.f = _hip.to_device(fpack, dt)
         self.U = torch.zeros(offk, dtype=dt, device="cuda")
         self.r = torch.zeros(offk, dtype=dt, device="cuda")
-        self.Ub = torch.zeros(offk, dtype=dt, device="cuda")
-        self.rb = torch.zeros(offk, dtype=dt, device="cuda")
         self.p = torch.zeros(2 * offk, dtype=dt, device="cuda")
         self.z = torch.zeros(2 * offk, dtype=dt, device="cuda")
+        # the one-pass iteration's second buffers of U, p and z; between its iterations they hold
+        # nothing, and the two-pass iteration keeps x_bar there
+        try:
+            self._other = tuple(torch.zeros_like(t) for t in (self.U, self.p, self.z))
+            self.Ub, self.rb = self._other[0], self._other[1][:offk]
+        except torch.cuda.OutOfMemoryError:  # a batch that only the two passes' buffers fit beside
+            self._other = None
+            self.Ub, self.rb = (torch.zeros(offk, dtype=dt, device="cuda") for _ in range(2))
         self.partials = torch.zeros(PARTIALS_PER_TILE * max(t0, 1), dtype=torch.float64, device="cuda")
         self.checks = torch.zeros(self.B * CHECK_DOUBLES, dtype=torch.float64, device="cuda")
         self.active_inst = torch.zeros(self.B, dtype=torch.int32, device="cuda")
@@ -150,7 +157,38 @@ class LiftBatch(object):
         if rc != 0:
             raise _hip.HipError("%s failed: %s" % (name, lib.opy_last_error().decode()))
 
+    def _one_pass(self):
+        """Whether iterations run in pairs of the one-pass kernel: up to 24
+        pieces (FP64: 16), and beyond where every instance has that many.  Its
+        LDS holds the largest piece count of the batch for every tile, so with
+        more than 24 two blocks fit a CU and a batch of mixed counts is faster
+        in two passes (3 to 30 pieces 157 against 171 us per iteration, 3 to 23
+        pieces 127 against 105, 32 pieces throughout 186 against 163)."""
+        if self._other is None:
+            return False
+        if self.dtype != torch.float32:
+            return self.kmax <= 16
+        return self.kmax <= 24 or min(self.K) > 24
+
+    def _iterations(self, n):
+        """n iterations from and to the buffers U, r, p, z: pairs through the
+        one-pass kernel, there and back between the two sets of buffers, and a
+        last odd one in place (an instance that has stopped is not written, so
+        its iterate must stay in the first set)."""
+        if self._one_pass():
+            Pt, s = _hip.ptr, _hip.stream()
+            ctl = (Pt(self.insts), Pt(self.active_inst), Pt(self.act_off), Pt(self.nact), self.kmax, self.grid, s)
+            a, b = (self.U, self.p, self.z), self._other
+            for _ in range(n // 2):
+                for i, o in ((a, b), (b, a)):
+                    self._call("opy_lift_iter" + self._sfx(), Pt(i[0]), Pt(o[0]), Pt(self.r), Pt(i[1]), Pt(o[1]),
+                               Pt(i[2]), Pt(o[2]), Pt(self.f), *ctl)
+            n %= 2
+        for _ in range(n):
+            self._iteration()
+
     def _iteration(self):
+        """One iteration in place, in two passes."""
         Pt, s = _hip.ptr, _hip.stream()
         ctl = (Pt(self.insts), Pt(self.active_inst), Pt(self.act_off), Pt(self.nact), self.kmax, self.grid, s)
         self._call("opy_lift_primal" + self._sfx(), Pt(self.U), Pt(self.r), Pt(self.Ub), Pt(self.rb), Pt(self.p),
@@ -246,16 +284,14 @@ class LiftBatch(object):
                 if key in graphs:
                     graphs[key].replay()
                 elif not warm:
-                    for _ in range(n):
-                        self._iteration()
+                    self._iterations(n)
                     torch.cuda.synchronize()
                     warm = True
                 else:
-                    graphs[key] = self._capture(lambda: [self._iteration() for _ in range(n)])
+                    graphs[key] = self._capture(lambda: self._iterations(n))
                     graphs[key].replay()
             else:
-                for _ in range(n):
-                    self._iteration()
+                self._iterations(n)
             done += n
             since += n
             nblk += 1

@@ -145,3 +145,34 @@ def test_lifting_primal_weight(gpu, fused):
     xo1, _, _, _ = opd.solve(prob, steps="precond", term_maxiter=80, granularity=80, term_pd_gap=1e-30)
     assert np.abs(x - xo).max() < 1e-9 and np.abs(y - yo).max() < 1e-9 * max(1.0, np.abs(yo).max())
     assert np.abs(xo - xo1).max() > 1e-3  # the weight changes the iterates
+
+
+@pytest.mark.parametrize("precision", ["double", "float"])
+@pytest.mark.parametrize("Ls", [[2, 3, 9, 5, 4], [10, 17, 2, 8, 13], [25, 18, 7, 24, 3], [26, 33, 27, 28, 30]])
+def test_one_pass_iteration_equals_two_passes(gpu, precision, Ls):
+    """The one-pass kernel against a primal and a dual pass, 5 iterations (two
+    pairs and an odd one) on images at the edges of its 64 x 4 tiles (one
+    pixel, one row or column more or less) with piece counts at the edges of
+    its instantiations.  Both form the same expressions; the tolerances leave
+    room for contractions (1e-12 FP64, 2e-5 FP32, of values up to ~10)."""
+    from opymize_amd.solvers.lift import LiftBatch
+    rng = np.random.default_rng(sum(Ls))
+    imgs = [rng.random(s) for s in ((4, 64), (5, 65), (1, 129), (9, 63), (7, 1))]
+    out = []
+    for one in (True, False):
+        lb = LiftBatch(imgs, Ls, [0.2, 0.1, 0.3, 0.15, 0.25], precision=precision, omega=3.0)
+        lb.reset()  # every instance running
+        # seven iterations in place first: a state with every kind of boundary active
+        for _ in range(7):
+            lb._iteration()
+        if one and precision == "double" and lb.kmax > 16:
+            assert not lb._one_pass()
+        if one:
+            lb._iterations(5)
+        else:
+            for _ in range(5):
+                lb._iteration()
+        out.append([t.cpu().numpy() for t in (lb.U, lb.r, lb.p, lb.z)])
+    tol = 1e-12 if precision == "double" else 2e-5
+    for a, b in zip(*out):
+        assert np.abs(b).max() > 0 and np.abs(a - b).max() <= tol * max(1.0, np.abs(b).max())
