@@ -286,6 +286,17 @@ int opy_pdhg_residual2_f64(const opy_step_t* a, const double* z, const double* z
  * OPY_RED_BLOCKS blocks.  Calls that overlap on one GPU race on that array.  Allocates nothing. */
 int opy_pdhg_residual2_noalloc_f32(const opy_step_t* a, const float* z, const float* zn, double b, const float* g,
                                    double c1, double c2, const float* gn, int64_t n, double* out2, void* stream);
+/* both residual sums of an iteration and the step rule (two opy_pdhg_residual2 calls into state->sums, then
+ * opy_pdhg_adapt, the same results): x, xn, A^T y and A^T y+ (n entries), y, y+, A x and A x+ (m entries);
+ * work: 4 * OPY_RED_BLOCKS doubles */
+int opy_pdhg_residuals_f32(const opy_step_t* tau, const float* x, const float* xn, const float* gx, const float* gxn,
+                           int64_t n, const opy_step_t* sigma, const float* y, const float* yn, double theta,
+                           const float* gy, const float* gyn, int64_t m, double* work, opy_adapt_state_t* state,
+                           const opy_adapt_params_t* params, void* stream);
+int opy_pdhg_residuals_f64(const opy_step_t* tau, const double* x, const double* xn, const double* gx,
+                           const double* gxn, int64_t n, const opy_step_t* sigma, const double* y, const double* yn,
+                           double theta, const double* gy, const double* gyn, int64_t m, double* work,
+                           opy_adapt_state_t* state, const opy_adapt_params_t* params, void* stream);
 /* adaptive step rule on the device; pdhg.py:166-183 */
 int opy_pdhg_adapt(opy_adapt_state_t* state, const opy_adapt_params_t* params, void* stream);
 

@@ -116,6 +116,7 @@ _SIGS = {
     "pdhg_take_step": [_P, _P, _L, _I, _P, _P, _P],
     "pdhg_dual_step": [_P, _P, _L, _D, _P, _P, _P, _P],
     "pdhg_residual2": [_P, _P, _P, _D, _P, _D, _D, _P, _L, _P, _P, _P],
+    "pdhg_residuals": [_P, _P, _P, _P, _P, _L, _P, _P, _P, _D, _P, _P, _L, _P, _P, _P, _P],
     "fn_eval": [_I, _P, _L, _I, _P, _P, _P, _I, _P],
     "clip": [_P, _P, _L, _D, _D, _P],
     "simplex_proj": [_P, _L, _I, _P],
@@ -299,6 +300,6 @@ class Workspace:
         dev = torch.cuda.current_device()
         b = cls._bufs.get(dev)
         if b is None:
-            b = torch.zeros(3 * OPY_RED_BLOCKS, dtype=torch.float64, device="cuda")
+            b = torch.zeros(4 * OPY_RED_BLOCKS, dtype=torch.float64, device="cuda")
             cls._bufs[dev] = b
         return b

@@ -200,6 +200,105 @@ __global__ void __launch_bounds__(kBlock) div2f_kernel(const T* __restrict__ p, 
   *out = add ? *out + val : val;
 }
 
+// The centered gradient and its adjoint on a 2-D grid, likewise: the terms of
+// grad_kernel<T, true> / div_kernel<T, true> in their order (the same bits),
+// every neighbour read once.  1024^2, C = 1, FP32: 12.8 -> 5.7 us and 18.0 ->
+// 5.5 us per call.
+template <typename T, int CT>
+__global__ void __launch_bounds__(kBlock) grad2c_kernel(const T* __restrict__ x, T* __restrict__ y, int H, int W,
+                                                        int Cr, const double* __restrict__ w, double h0, double h1,
+                                                        int add) {
+  const int C = CT > 0 ? CT : Cr;
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= W * C) return;
+  const int r = blockIdx.y;
+  const int c = e / C;
+  const int k = e - c * C;
+  const int i = r * W + c;
+  const double wk = w ? w[k] : 1.0;
+  T v0 = T(0), v1 = T(0);
+  if (r < H - 1 && c < W - 1) {
+    const T a = x[i * C + k], b = x[(i + 1) * C + k], d = x[(i + W) * C + k], f = x[(i + W + 1) * C + k];
+    v0 = (T)(wk / (h0 * 2.0)) * ((d - a) + (f - b));
+    v1 = (T)(wk / (h1 * 2.0)) * ((b - a) + (f - d));
+  }
+  if constexpr (CT == 1) {
+    using V2 = typename Vec2<T>::type;
+    V2* out = reinterpret_cast<V2*>(y) + i;
+    V2 o;
+    if (add) {
+      o = *out;
+      o.x += v0;
+      o.y += v1;
+    } else {
+      o.x = v0;
+      o.y = v1;
+    }
+    *out = o;
+  } else {
+    T* out = y + (i * 2) * C + k;
+    out[0] = add ? out[0] + v0 : v0;
+    out[C] = add ? out[C] + v1 : v1;
+  }
+}
+
+template <typename T, int CT>
+__global__ void __launch_bounds__(kBlock) div2c_kernel(const T* __restrict__ p, T* __restrict__ x, int H, int W,
+                                                       int Cr, const double* __restrict__ w, double h0, double h1,
+                                                       int add) {
+  const int C = CT > 0 ? CT : Cr;
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= W * C) return;
+  const int r = blockIdx.y;
+  const int c = e / C;
+  const int k = e - c * C;
+  const int i = r * W + c;
+  const double wk = w ? w[k] : 1.0;
+  const T ih0 = (T)(1.0 / h0), ih1 = (T)(1.0 / h1);
+  // p at the point and at its neighbours up and left
+  T q[2][2][2];  // [row - 1, row][column - 1, column][axis]
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      q[a][b][0] = q[a][b][1] = T(0);
+      const bool in = (a == 1 || r > 0) && (b == 1 || c > 0);
+      const int j = i - (1 - a) * W - (1 - b);
+      if (in) {
+        if constexpr (CT == 1) {
+          using V2 = typename Vec2<T>::type;
+          const V2 v = reinterpret_cast<const V2*>(p)[j];
+          q[a][b][0] = v.x;
+          q[a][b][1] = v.y;
+        } else {
+          q[a][b][0] = p[(j * 2) * C + k];
+          q[a][b][1] = p[(j * 2 + 1) * C + k];
+        }
+      }
+    }
+  const bool dn = r < H - 1, up = r > 0, rt = c < W - 1, lf = c > 0;
+  T acc = T(0);
+  if (rt) {
+    if (dn) acc -= q[1][1][0] * ih0;
+    if (up) acc += q[0][1][0] * ih0;
+  }
+  if (lf) {
+    if (dn) acc -= q[1][0][0] * ih0;
+    if (up) acc += q[0][0][0] * ih0;
+  }
+  if (dn) {
+    if (rt) acc -= q[1][1][1] * ih1;
+    if (lf) acc += q[1][0][1] * ih1;
+  }
+  if (up) {
+    if (rt) acc -= q[0][1][1] * ih1;
+    if (lf) acc += q[0][0][1] * ih1;
+  }
+  const T val = (T)(wk / 2.0) * acc;
+  T* out = x + i * C + k;
+  *out = add ? *out + val : val;
+}
+
 // The same on a 3-D grid (d0 x d1 x d2): a thread per (i1, i2, channel) of
 // slab i0 = blockIdx.y, with 32-bit index arithmetic (the lifting model's
 // (H, W, labels) grid, whose label axis is short).
@@ -275,7 +374,7 @@ inline bool use_3d_forward(const Grid& g) {
 
 // The 2-D kernels serve forward 2-D grids whose indices fit 32 bits and whose
 // rows fit the grid's second dimension.
-inline bool use_2d_forward(const Grid& g) {
+inline bool use_2d(const Grid& g) {
   return g.ndims == 2 && g.dims[0] >= 1 && g.dims[0] <= 65535 && g.npoints * g.nchan * 2 < (int64_t(1) << 31);
 }
 
@@ -527,9 +626,12 @@ int grad_impl(const T* x, T* y, const opy_grid_t* gd, const double* w, int schem
   if (int rc = make_grid(gd, &g)) return rc;
   if (!x || !y) return fail(kInvalid, "gradient: null pointer");
   const int64_t n = g.npoints * g.nchan;
-  if (scheme == OPY_SCHEME_CENTERED)
+  if (scheme == OPY_SCHEME_CENTERED && use_2d(g)) {
+    if (n > 0) OPY_LAUNCH_2F(grad2c_kernel, T, x, y, g, w, add, as_stream(s),
+                             reinterpret_cast<uintptr_t>(y) % (2 * sizeof(T)) == 0);
+  } else if (scheme == OPY_SCHEME_CENTERED)
     hipLaunchKernelGGL((grad_kernel<T, true>), dim3(grid_for(n)), dim3(kBlock), 0, as_stream(s), x, y, g, w, add);
-  else if (scheme == OPY_SCHEME_FORWARD && use_2d_forward(g)) {
+  else if (scheme == OPY_SCHEME_FORWARD && use_2d(g)) {
     if (n > 0) OPY_LAUNCH_2F(grad2f_kernel, T, x, y, g, w, add, as_stream(s),
                              reinterpret_cast<uintptr_t>(y) % (2 * sizeof(T)) == 0);
   } else if (scheme == OPY_SCHEME_FORWARD && use_3d_forward(g)) {
@@ -547,9 +649,12 @@ int div_impl(const T* p, T* x, const opy_grid_t* gd, const double* w, int scheme
   if (int rc = make_grid(gd, &g)) return rc;
   if (!x || !p) return fail(kInvalid, "divergence: null pointer");
   const int64_t n = g.npoints * g.nchan;
-  if (scheme == OPY_SCHEME_CENTERED)
+  if (scheme == OPY_SCHEME_CENTERED && use_2d(g)) {
+    if (n > 0) OPY_LAUNCH_2F(div2c_kernel, T, p, x, g, w, add, as_stream(s),
+                             reinterpret_cast<uintptr_t>(p) % (2 * sizeof(T)) == 0);
+  } else if (scheme == OPY_SCHEME_CENTERED)
     hipLaunchKernelGGL((div_kernel<T, true>), dim3(grid_for(n)), dim3(kBlock), 0, as_stream(s), p, x, g, w, add);
-  else if (scheme == OPY_SCHEME_FORWARD && use_2d_forward(g)) {
+  else if (scheme == OPY_SCHEME_FORWARD && use_2d(g)) {
     if (n > 0) OPY_LAUNCH_2F(div2f_kernel, T, p, x, g, w, add, as_stream(s),
                              reinterpret_cast<uintptr_t>(p) % (2 * sizeof(T)) == 0);
   } else if (scheme == OPY_SCHEME_FORWARD && use_3d_forward(g)) {

@@ -241,17 +241,11 @@ class PDHG(object):
 
         if "adaptive" in c:
             adapt = d["adapt"]
-            work = _hip.Workspace.get()
-            sums = _hip.addr(adapt, _hip.ADAPT_FIELD["sums"])
-            sums2 = _hip.addr(adapt, _hip.ADAPT_FIELD["sums"] + 2)
-            st = _hip.make_step(tau, dtype)
-            _hip.call("pdhg_residual2", dtype, _hip.ctypes.byref(st), _hip.ptr(xk), _hip.ptr(xkp1), 1.0,
-                      _hip.ptr(xgradk), 1.0, 0.0, _hip.ptr(xgradkp1), xk.numel(), _hip.ptr(work), sums, stream)
-            ss = _hip.make_step(sigma, dtype)
-            _hip.call("pdhg_residual2", dtype, _hip.ctypes.byref(ss), _hip.ptr(yk), _hip.ptr(ykp1), float(theta),
-                      _hip.ptr(ygradk), float(theta), float(theta) + 1.0, _hip.ptr(ygradkp1), yk.numel(),
-                      _hip.ptr(work), sums2, stream)
-            _hip.call_plain("opy_pdhg_adapt", _hip.ptr(adapt), _hip.ctypes.byref(self._adapt_params), stream)
+            st, ss = _hip.make_step(tau, dtype), _hip.make_step(sigma, dtype)
+            _hip.call("pdhg_residuals", dtype, _hip.ctypes.byref(st), _hip.ptr(xk), _hip.ptr(xkp1), _hip.ptr(xgradk),
+                      _hip.ptr(xgradkp1), xk.numel(), _hip.ctypes.byref(ss), _hip.ptr(yk), _hip.ptr(ykp1),
+                      float(theta), _hip.ptr(ygradk), _hip.ptr(ygradkp1), yk.numel(), _hip.ptr(_hip.Workspace.get()),
+                      _hip.ptr(adapt), _hip.ctypes.byref(self._adapt_params), stream)
             if not self._adapt_dev_steps:
                 self._sync_host_steps()
 

@@ -415,3 +415,57 @@ def test_indexedmult_refuses_bad_indices(gpu):
         IndexedMult(4, 10, np.ones((2, 1, 3)), np.array([[0, 1, 4], [0, 0, 0]]))
     with pytest.raises(ValueError):
         IndexedMult(4, 10, np.ones((2, 1, 3)), np.zeros((2, 2), dtype=int))
+
+
+@pytest.mark.parametrize("dims", [(1, 1), (1, 5), (6, 1), (2, 2), (3, 257), (259, 4), (31, 64)])
+@pytest.mark.parametrize("C", [1, 2, 3])
+def test_centered_2d_at_edges(gpu, dims, C):
+    """The 2-D kernels of the centered gradient and its adjoint against the
+    sparse matrix, with and without accumulation, at one-row, one-column and
+    block-edge sizes (FP64, 1e-13 of values of size 1)."""
+    import torch
+    from opymize_amd.linear import GradientOp
+    from oracle import ops
+    rng = np.random.default_rng(dims[0] * 7 + dims[1] + C)
+    h, w = (0.5, 2.0), np.arange(1, C + 1) * 0.75
+    A = GradientOp(dims, C, scheme="centered", imageh=h, weights=w)
+    M = ops.grad_matrix(dims, C, h=np.array(h), w=w, scheme="centered")
+    x, y = rng.standard_normal(A.x.size), rng.standard_normal(A.y.size)
+    dev = lambda a: torch.as_tensor(a).cuda()  # noqa: E731
+    for op, mat, a, b in ((A, M, x, y), (A.adjoint, M.T, y, x)):
+        for add in (False, True):
+            out = dev(b.copy())
+            op(dev(a), out, add=add)
+            ref = mat @ a + (b if add else 0.0)
+            assert np.abs(out.cpu().numpy() - ref).max() <= 1e-13 * max(1.0, np.abs(ref).max())
+
+
+@pytest.mark.parametrize("n,m", [(1, 2), (257, 512), (300000, 600001)])
+def test_residuals_in_one_call_equal_the_separate_ones(gpu, n, m):
+    """opy_pdhg_residuals against two opy_pdhg_residual2 calls and
+    opy_pdhg_adapt: the same bits in the whole state (fewer elements than a
+    block, one block's, and more than the grid's)."""
+    import torch
+    from opymize_amd import _hip
+    gen = torch.Generator("cuda").manual_seed(n)
+    x = [torch.randn(n, generator=gen, device="cuda") for _ in range(4)]
+    y = [torch.randn(m, generator=gen, device="cuda") for _ in range(4)]
+    F = _hip.ADAPT_FIELD
+    st = torch.zeros(_hip.ADAPT_STATE_DOUBLES, dtype=torch.float64)
+    st[F["tau"]], st[F["sigma"]], st[F["alpha"]] = 0.3, 0.2, 0.5
+    p = _hip.AdaptParams()
+    p.eta, p.Delta, p.sqrt_n, p.sqrt_m = 0.95, 1.5, n ** 0.5, m ** 0.5
+    p.eps_absp = p.eps_relp = p.eps_absd = p.eps_reld = 1e-4
+    a, b = st.cuda(), st.cuda()
+    P, s, by = _hip.ptr, _hip.stream(), _hip.ctypes.byref
+    work = _hip.Workspace.get()
+    tau, sig = _hip.make_step((a, F["tau"]), torch.float32), _hip.make_step((a, F["sigma"]), torch.float32)
+    _hip.call("pdhg_residual2", torch.float32, by(tau), P(x[0]), P(x[1]), 1.0, P(x[2]), 1.0, 0.0, P(x[3]), n, P(work),
+              _hip.addr(a, F["sums"]), s)
+    _hip.call("pdhg_residual2", torch.float32, by(sig), P(y[0]), P(y[1]), 1.0, P(y[2]), 1.0, 2.0, P(y[3]), m, P(work),
+              _hip.addr(a, F["sums"] + 2), s)
+    _hip.call_plain("opy_pdhg_adapt", P(a), by(p), s)
+    tau, sig = _hip.make_step((b, F["tau"]), torch.float32), _hip.make_step((b, F["sigma"]), torch.float32)
+    _hip.call("pdhg_residuals", torch.float32, by(tau), P(x[0]), P(x[1]), P(x[2]), P(x[3]), n, by(sig), P(y[0]),
+              P(y[1]), 1.0, P(y[2]), P(y[3]), m, P(work), P(b), by(p), s)
+    assert torch.equal(a.view(torch.int64), b.view(torch.int64))
