@@ -189,11 +189,17 @@ def sfx(dtype):
     raise TypeError("opymize_amd kernels support float32 and float64, got %s" % dtype)
 
 
+_fns = {}  # (name, dtype) -> bound entry point
+
+
 def call(name, dtype, *args):
     """Call opy_<name>_<f32|f64>(*args) and raise HipError on failure."""
-    lib = load()
-    fname = "opy_%s%s" % (name, sfx(dtype))
-    _check(getattr(lib, fname)(*args), fname)
+    fn = _fns.get((name, dtype))
+    if fn is None:
+        fn = _fns[(name, dtype)] = getattr(load(), "opy_%s%s" % (name, sfx(dtype)))
+    rc = fn(*args)
+    if rc != 0:
+        _check(rc, "opy_%s%s" % (name, sfx(dtype)))
 
 
 def call_plain(name, *args):
@@ -202,8 +208,9 @@ def call_plain(name, *args):
 
 
 def stream():
-    """Handle of torch's current stream on the current device."""
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """Handle of torch's current stream on the current device (the raw handle:
+    a torch.cuda.Stream object costs more than a small launch)."""
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def require_device():
@@ -219,6 +226,8 @@ def ptr(t, dtype=None, numel=None):
     """Device pointer of a contiguous CUDA tensor (None -> NULL)."""
     if t is None:
         return None
+    if dtype is None and numel is None and type(t) is torch.Tensor and t.is_cuda and t.is_contiguous():
+        return ctypes.c_void_p(t.data_ptr())
     if not isinstance(t, torch.Tensor) or not t.is_cuda:
         raise TypeError("expected a ROCm device tensor, got %r" % type(t))
     if not t.is_contiguous():

@@ -22,8 +22,14 @@ def _check_pair(x, y, nx, ny, what):
 
 
 class _DiffBase(LinOp):
+    _grid_of = (None, None)
+
     def _grid(self):
-        return _hip.make_grid(self.imagedims, self.nchannels, self.imageh)
+        """The grid description, built again only when an attribute it is made of has changed."""
+        key = (tuple(self.imagedims), self.nchannels, self.imageh.tobytes())
+        if self._grid_of[0] != key:
+            self._grid_of = (key, _hip.make_grid(self.imagedims, self.nchannels, self.imageh))
+        return self._grid_of[1]
 
     def _w(self):
         return self._const.get("weights", np.asarray(self.weights, dtype=np.float64), _hip.torch_dtype("double"))
