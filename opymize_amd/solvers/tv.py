@@ -254,7 +254,9 @@ class TVBatch(object):
         self.set_stream_rows(stream_rows)
         self.set_tile(*tile)
         self.graph = None
-        self.cur = 0  # buffer holding the current iterate
+        self.cur = 0  # buffer holding the current iterate of the running instances
+        self._running_now = np.ones(self.B, dtype=bool)
+        self._stopped_in = np.zeros(self.B, dtype=np.int8)  # a stopped instance's buffer
         self._restart = None  # (beta, min_iters, tau0, sigma0) while a solve restarts its schedule
 
     # -- layout --------------------------------------------------------------
@@ -420,6 +422,10 @@ class TVBatch(object):
         run = self._running.cpu().numpy()
         nrun = int(run[0])
         running = run[1:1 + nrun]
+        now = np.zeros(self.B, dtype=bool)
+        now[running] = True
+        self._stopped_in[self._running_now & ~now] = self.cur
+        self._running_now = now
         self.grid = self._launch_grid(int(run[self.B + 1 + nrun]))
         if self.multi > 1:
             units = int(np.sum(self._strips[running] * -(-self._H[running] // self.stream_rows)))
@@ -619,11 +625,21 @@ class TVBatch(object):
             self.cur = end
 
     def _to_buffer0(self):
-        """Bring the current iterate to buffer 0 (the start and result buffer)."""
-        if self.cur != 0:
+        """Bring each instance's iterate to buffer 0 (the start and result
+        buffer).  Launches leave a stopped instance alone, so its iterate stays
+        in the buffer that was current at its last check, which an odd number
+        of launches per block makes another one than the running instances'."""
+        inst = np.where(self._running_now, self.cur, self._stopped_in)
+        if inst.all():
             for a in (self.x, self.y):
                 _hip.call("copy", self.dtype, _hip.ptr(a[1]), _hip.ptr(a[0]), a[0].numel(), _hip.stream())
-            self.cur = 0
+        else:
+            for b in np.flatnonzero(inst):
+                n, off = int(self._H[b] * self._W[b]) * self.C, int(self.offs[b])
+                self.x[0][off:off + n].copy_(self.x[1][off:off + n])
+                self.y[0][2 * off:2 * off + 2 * n].copy_(self.y[1][2 * off:2 * off + 2 * n])
+        self._stopped_in[:] = 0
+        self.cur = 0
 
     @staticmethod
     def _capture(fn):
@@ -725,6 +741,7 @@ class TVBatch(object):
             sigma0 = np.sqrt(step_bound / restart_factor)  # TV-L2 instances only restart
             self._restart = (float(beta), int(min_iters), step_bound / sigma0, sigma0)
         self.cur = 0
+        self._running_now[:], self._stopped_in[:] = True, 0
         if check_start:
             self._check_step(cfg, tol, tol_infeas, certify, 0)
             if fallback:
@@ -798,5 +815,9 @@ class TVBatch(object):
                 for b in range(self.B)]
 
     def solution(self):
-        """Per-instance (x, y) host arrays of the current iterates (buffer 0)."""
-        return self.unpack(self.x[self.cur], "x"), self.unpack(self.y[self.cur], "y")
+        """Per-instance (x, y) host arrays of the current iterates."""
+        inst = np.where(self._running_now, self.cur, self._stopped_in)
+        if not inst.any():
+            return self.unpack(self.x[0], "x"), self.unpack(self.y[0], "y")
+        both = [[self.unpack(a[p], f) for p in (0, 1)] for a, f in ((self.x, "x"), (self.y, "y"))]
+        return tuple([v[inst[b]][b] for b in range(self.B)] for v in both)

@@ -78,6 +78,30 @@ def test_wide_graph_replays_equal_eager(gpu):
         np.testing.assert_array_equal(a, b)
 
 
+@pytest.mark.parametrize("kernel", ["auto", "stream"])
+@pytest.mark.parametrize("graph", [True, False])
+def test_stopped_instances_keep_their_iterate_over_odd_blocks(gpu, graph, kernel):
+    """Three launches of 8 iterations per block: the buffers change places
+    at every check, and an instance certified at one of them keeps the iterate
+    that was certified, whichever buffer later blocks end in (single launches
+    as the reference, bit for bit)."""
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
+    out = []
+    for multi in (8, 1):
+        bat = tv.TVBatch(imgs, [2.0, 9.0, 15.0, 19.0], "l2", multi=multi, multi_kernel=kernel)
+        bat.stream_min_units = 0
+        mid = []
+        res = bat.solve(steps="accel", step_bound=0.124, step_factor=4.0, max_iters=2400, block_iters=24, tol=1e-5,
+                        use_graph=graph, callback=lambda b, n: mid.append(b.solution()[0][0]) if n <= 240 else None)
+        out.append(([(r["iter"], r["gap"], r["status"]) for r in res], bat.solution(), mid))
+    its = [i // 24 for i, _, s in out[0][0]]
+    assert len(set(i % 2 for i in its)) == 2  # stopped in different buffers
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1][0] + out[0][1][1] + out[0][2], out[1][1][0] + out[1][1][1] + out[1][2]):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_wide_entry_points_refuse_bad_arguments():
     """Host checks before any launch."""
     import ctypes
