@@ -131,8 +131,11 @@ def _wide_strips(W, sw):
     return np.minimum(-(-W // sw), np.where(W <= WIDE_COLS, 1, -(-(W - WIDE_COLS) // sw) + 1))
 
 
+# iterations per streaming launch from which blocks run without a graph (_captured)
+CAPTURE_BELOW = 4
+
 # rows per unit that the two-column kernel may take (wide_rows)
-WIDE_ROWS = (8, 10, 12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 52, 57, 64, 69, 74, 80, 86, 94, 103, 114, 128,
+WIDE_ROWS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 52, 57, 64, 69, 74, 80, 86, 94, 103, 114, 128,
              147, 171, 205, 256, 342, 512)
 
 
@@ -146,7 +149,11 @@ def wide_rows(H, strips, k, simds):
     takes 0.95 of, and those left over when the others have ended leave most
     of the chip idle.  (Microseconds per row step, measured at 8 iterations
     per launch on 32 and 128 images of 1024^2 with 48 to 256 rows: within 10%
-    of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)"""
+    of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)
+    Where every unit has a SIMD of its own the shortest units win, down to
+    one row each (960 iterations of one 64^2 image: 8 rows 3.73 ms, 4 rows
+    3.34, 1 row 3.01; of one 512^2 image 3.79, 3.38 and, past a unit per SIMD,
+    5.65)."""
     best, rows = None, WIDE_ROWS[-1]
     for R in WIDE_ROWS:
         chunks = -(-H // R)
@@ -154,7 +161,9 @@ def wide_rows(H, strips, k, simds):
         n = float(np.sum(units))
         steps = float(np.sum(units * (-(-H // chunks) + 2 * k))) / n  # of a unit, on average
         rounds, rest = divmod(n / simds, 2.0)
-        cost = steps * (1.54 * rounds + (0.0 if rest < 0.01 else 0.95 if rest <= 1.0 else 1.54))
+        if rounds and rest < 0.01:
+            rest = 0.0  # a handful of units beside the full rounds
+        cost = steps * (1.54 * rounds + (0.0 if rest == 0.0 else 0.95 if rest <= 1.0 else 1.54))
         if best is None or cost < best:
             best, rows = cost, R
     return rows
@@ -624,6 +633,18 @@ class TVBatch(object):
             g.replay()
             self.cur = end
 
+    def _captured(self, cfg, adapt):
+        """Whether blocks of launches are worth a captured graph.  A capture
+        costs 0.3 to 0.4 ms and the replay after each check's read starts 10 us
+        later than plain launches, which single iterations (a few us each) earn
+        back and the streaming kernels' launches, longer than the host takes
+        to issue the next, do not: per 480 and 4800 iterations in blocks of 48,
+        captured against plain, one image of 64^2 takes 2.9 / 18.4 against 2.6 /
+        25.3 ms at 2 iterations per launch, 2.5 / 17.7 against 1.8 / 16.1 at 4 and
+        2.7 / 20.8 against 2.1 / 19.1 at 8, one of 1024^2 3.3 / 26.7 against 2.7 /
+        24.9 at 8."""
+        return adapt or self._launch_k(cfg) < CAPTURE_BELOW or not (self._use_wide(cfg) or self._use_stream(cfg))
+
     def _to_buffer0(self):
         """Bring each instance's iterate to buffer 0 (the start and result
         buffer).  Launches leave a stopped instance alone, so its iterate stays
@@ -756,14 +777,15 @@ class TVBatch(object):
                 return self.results()
         else:
             self.refresh_grid()
-        graphs = use_graph
+        def graphs():
+            return use_graph and self._captured(cfg, adapt)
         # captured blocks per (launch grid, buffer holding the iterate at the start)
         g_it, g_ck = {"warm": False}, {"warm": False}
         done_iters, nblk = 0, 0
         since = 0
         while done_iters < max_iters:
             n = min(block_iters, max_iters - done_iters)
-            if graphs and n == block_iters:
+            if n == block_iters and graphs():
                 self._graph_block(g_it, lambda: self._iterations(n, cfg, adapt, params))
             else:
                 self._iterations(n, cfg, adapt, params)
@@ -771,7 +793,7 @@ class TVBatch(object):
             since += n
             nblk += 1
             if nblk % check_every == 0 or done_iters >= max_iters:
-                if graphs and since == block_iters * check_every:
+                if since == block_iters * check_every and graphs():
                     self._graph_block(g_ck, lambda: self._check_step(cfg, tol, tol_infeas, certify,
                                                                      block_iters * check_every))
                 else:

@@ -30,7 +30,8 @@ def _run(multi, kernel, steps, rows, monkeypatch, shapes=SHAPES, iters=24):
 
 
 @pytest.mark.parametrize("steps", ["accel", "const"])
-@pytest.mark.parametrize("multi,rows", [(2, 8), (3, 40), (4, 8), (5, 256), (6, 32), (7, 8), (8, 8), (8, 40), (8, 256)])
+@pytest.mark.parametrize("multi,rows", [(2, 8), (3, 40), (4, 8), (5, 256), (6, 32), (7, 8), (8, 8), (8, 40), (8, 256),
+                                        (2, 1), (4, 3), (8, 1), (8, 2)])
 def test_wide_equals_single_launches(gpu, monkeypatch, multi, rows, steps):
     """Two blocks of a whole number of launches and a remainder of single
     iterations (25 = 3 * 8 + 1), TV-L1 and TV-L2, uneven TV weights."""
@@ -62,10 +63,11 @@ def test_wide_units_follow_the_running_instances(gpu):
         np.testing.assert_array_equal(off.cpu().numpy()[:nrun + 1], np.concatenate([[0], np.cumsum(counts)]))
 
 
-def test_wide_graph_replays_equal_eager(gpu):
+def test_wide_graph_replays_equal_eager(gpu, monkeypatch):
     """Captured blocks (the step table among them) replayed many times against
     eager launches, on a batch that certifies instance by instance."""
     from opymize_amd.solvers import tv
+    monkeypatch.setattr(tv, "CAPTURE_BELOW", 9)  # capture at 8 iterations per launch too
     imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
     out = []
     for g in (True, False):
@@ -80,12 +82,13 @@ def test_wide_graph_replays_equal_eager(gpu):
 
 @pytest.mark.parametrize("kernel", ["auto", "stream"])
 @pytest.mark.parametrize("graph", [True, False])
-def test_stopped_instances_keep_their_iterate_over_odd_blocks(gpu, graph, kernel):
+def test_stopped_instances_keep_their_iterate_over_odd_blocks(gpu, monkeypatch, graph, kernel):
     """Three launches of 8 iterations per block: the buffers change places
     at every check, and an instance certified at one of them keeps the iterate
     that was certified, whichever buffer later blocks end in (single launches
     as the reference, bit for bit)."""
     from opymize_amd.solvers import tv
+    monkeypatch.setattr(tv, "CAPTURE_BELOW", 9)
     imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
     out = []
     for multi in (8, 1):
