@@ -154,19 +154,15 @@ def wide_rows(H, strips, k, simds):
     one row each (960 iterations of one 64^2 image: 8 rows 3.73 ms, 4 rows
     3.34, 1 row 3.01; of one 512^2 image 3.79, 3.38 and, past a unit per SIMD,
     5.65)."""
-    best, rows = None, WIDE_ROWS[-1]
-    for R in WIDE_ROWS:
-        chunks = -(-H // R)
-        units = strips * chunks
-        n = float(np.sum(units))
-        steps = float(np.sum(units * (-(-H // chunks) + 2 * k))) / n  # of a unit, on average
-        rounds, rest = divmod(n / simds, 2.0)
-        if rounds and rest < 0.01:
-            rest = 0.0  # a handful of units beside the full rounds
-        cost = steps * (1.54 * rounds + (0.0 if rest == 0.0 else 0.95 if rest <= 1.0 else 1.54))
-        if best is None or cost < best:
-            best, rows = cost, R
-    return rows
+    R = np.asarray(WIDE_ROWS)[:, None]
+    chunks = -(-H // R)
+    units = strips * chunks
+    n = units.sum(axis=1)
+    steps = (units * (-(-H // chunks) + 2 * k)).sum(axis=1) / n  # of a unit, on average
+    rounds, rest = np.divmod(n / simds, 2.0)
+    rest = np.where((rounds > 0) & (rest < 0.01), 0.0, rest)  # a handful of units beside the full rounds
+    cost = steps * (1.54 * rounds + np.where(rest == 0.0, 0.0, np.where(rest <= 1.0, 0.95, 1.54)))
+    return int(R[np.argmin(cost), 0])
 
 
 def tile_height(tw, rpt):
@@ -316,6 +312,8 @@ class TVBatch(object):
         set in steps of a sixteenth of the batch, so that a solve needs few
         distinct launch shapes (one captured graph each); blocks past the
         running units return at once."""
+        if self.C != 1 or self.dtype != torch.float32:
+            return False
         strips = _wide_strips(self._W, WIDE_COLS - 2 * self.multi)
         work = strips * self._H
         share = -(-16 * int(work[running].sum()) // int(work.sum())) if len(running) else 0
