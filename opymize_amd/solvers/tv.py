@@ -191,7 +191,8 @@ class TVBatch(object):
             stream_rows rows, the K iterations pipelined down the rows), "tile"
             (LDS-staged tiles, K <= 4), or "auto": one-channel FP32 batches
             stream strips of 128 - 2K columns, two per lane, whose rows per
-            unit follow from the running instances (wide_rows); others stream
+            unit follow from the running instances (wide_rows; large batches
+            with K < 6 excepted, _use_wide); others stream
             while the running instances give at least stream_min_units units
             (decided at each check), else take tiles with min(K, 4) iterations
             per launch; preconditioned steps take tiles.  Every choice gives
@@ -254,7 +255,7 @@ class TVBatch(object):
         # "auto" streams while the running instances give at least this many
         # units (about four wavefronts per SIMD), else takes the tile kernel
         self.stream_min_units = STREAM_MIN_UNITS
-        self._stream_now = True
+        self._stream_now = self._wide_now = True
         self.set_multi(multi)
         self.set_stream_rows(stream_rows)
         self.set_tile(*tile)
@@ -353,7 +354,16 @@ class TVBatch(object):
         return self.multi_kernel == "stream" or self._stream_now
 
     def _use_wide(self, cfg):
-        """Whether the next K-iteration launches run the two-column streaming kernel."""
+        """Whether the next K-iteration launches run the two-column streaming
+        kernel.  Below 6 iterations per launch a batch with more than 8192 of
+        the one-column kernel's units is left to that one: both wait for HBM
+        there, and it has twice the wavefronts to wait with (240 iterations of
+        128 images of 1024^2 with 2, 4, 5 per launch: one column 114, 55.2,
+        47.9 ms, two columns 119, 57.9, 48.6; with 6 40.6 against 39.2; of 32
+        images 27.0, 13.1, 11.5 against 25.6, 12.6, 11.2)."""
+        return self._wide_fits(cfg) and self._wide_now
+
+    def _wide_fits(self, cfg):
         return (self.multi_kernel == "auto" and self.multi > 1 and self.C == 1 and self.dtype == torch.float32
                 and cfg.steps != STEP_MODES["precond"] and self._stream_fits())
 
@@ -439,6 +449,7 @@ class TVBatch(object):
             if self._grid_override is None:
                 self.sgrid = self._stream_grid(units)
             self._stream_now = units >= self.stream_min_units
+            self._wide_now = self.multi >= 6 or units < 2 * STREAM_MIN_UNITS
             if self._size_wide(running):
                 self._stream_units()
         return nrun
@@ -565,13 +576,16 @@ class TVBatch(object):
         if cfg.steps == STEP_MODES["accel"]:
             self._call("opy_tv_accel_n", P(self.insts), P(self.state), P(self.checks), self.B, int(k), s)
 
+    def _wide_alloc(self):
+        if self._wide_table is None:
+            self._wide_table = torch.zeros(self.B * WIDE_TABLE * 8, dtype=torch.float32, device="cuda")
+
     def _wide_iterations(self, n, cfg, k):
         """The first n - n % k of n iterations on the two-column streaming
         kernel, k per launch; returns n % k."""
         P = _hip.ptr
         s = _hip.stream()
-        if self._wide_table is None:
-            self._wide_table = torch.zeros(self.B * WIDE_TABLE * 8, dtype=torch.float32, device="cuda")
+        self._wide_alloc()
         while n >= k:
             m = min(n, WIDE_TABLE)
             m -= m % k
@@ -614,7 +628,7 @@ class TVBatch(object):
         block of a solve runs eagerly, which loads its kernels before any
         capture; a new key is captured (that records without running) and
         then replayed."""
-        key = (self.grid, self.sgrid, self._stream_now, self.wrows, self.wgrid, self.cur)
+        key = (self.grid, self.sgrid, self._stream_now, self._wide_now, self.wrows, self.wgrid, self.cur)
         if key in cache:
             g, end = cache[key]
             g.replay()
@@ -775,6 +789,9 @@ class TVBatch(object):
                 return self.results()
         else:
             self.refresh_grid()
+        if self._wide_fits(cfg):
+            self._wide_alloc()  # before any block is captured
+
         def graphs():
             return use_graph and self._captured(cfg, adapt)
         # captured blocks per (launch grid, buffer holding the iterate at the start)

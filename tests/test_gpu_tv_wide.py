@@ -42,6 +42,27 @@ def test_wide_equals_single_launches(gpu, monkeypatch, multi, rows, steps):
     assert gaps == gaps1
 
 
+def test_kernel_may_change_between_blocks(gpu, monkeypatch):
+    """Fewer than 6 iterations per launch: one column per lane while the batch
+    is large, two from the check on at which enough instances stopped; captured
+    blocks and the iterates of single launches, bit for bit."""
+    from opymize_amd.solvers import tv
+    monkeypatch.setattr(tv, "STREAM_MIN_UNITS", 3)
+    imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
+    out = []
+    for multi in (3, 1):
+        bat = tv.TVBatch(imgs, [2.0, 9.0, 15.0, 19.0], "l2", multi=multi)
+        used = []
+        res = bat.solve(steps="accel", step_bound=0.124, step_factor=4.0, max_iters=4800, block_iters=48, tol=1e-5,
+                        callback=lambda b, n: used.append(b._wide_now))
+        out.append(([(r["iter"], r["gap"], r["status"]) for r in res], bat.solution()))
+        if multi > 1:
+            assert not used[0] and True in used
+    assert out[0][0] == out[1][0]
+    for a, b in zip(out[0][1][0] + out[0][1][1], out[1][1][0] + out[1][1][1]):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_wide_units_follow_the_running_instances(gpu):
     """The device's unit prefixes against a host recount, after some
     instances stopped; rows chosen for the whole and the reduced set."""
