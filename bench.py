@@ -27,10 +27,10 @@ Printed next to it:
     instances spread over the lambda range of the same batch, and the same
     instances one at a time through the batched solver's own kernels and
     step rule (so that ratio isolates the gain of batching);
-  * the roofline of the dominant kernel (by default the streaming kernel
-    that runs K = 8 iterations per launch, one wavefront per strip of 48
-    columns by 128 rows, the iterations pipelined down the rows; --multi-kernel
-    tile: the LDS-tile kernel, K <= 4; the single-pass iteration kernel with
+  * the roofline of the dominant kernel (by default the two-column streaming
+    kernel that runs K = 8 iterations per launch, one wavefront per strip of
+    112 columns, two per lane, the iterations pipelined down the rows;
+    --multi-kernel stream: one column per lane, strips of 48; tile: the LDS-tile kernel, K <= 4; the single-pass iteration kernel with
     --multi 1 or adaptive steps; the dual pass with --passes 2): algorithmic
     bytes of a full-batch launch over the average duration of eager
     full-batch launches, timed with HIP events on the launch stream; with
@@ -98,7 +98,11 @@ def roofline_phase(bat, reps, rule):
     s = _hip.stream()
 
     def launch(name):
-        if name == "multi" and bat._use_stream(cfg):
+        if name == "multi" and bat._use_wide(cfg):
+            bat._call("opy_tv_wide_f32", P(bat.x[0]), P(bat.x[1]), P(bat.y[0]), P(bat.y[1]), P(bat.f), P(bat.insts),
+                      P(table), tlen, 0, P(bat.active_inst), P(bat.wide_off), P(bat.nact), bat.multi, bat.wrows,
+                      bat.wgrid, s)
+        elif name == "multi" and bat._use_stream(cfg):
             bat._call("opy_tv_stream" + sfx, P(bat.x[0]), P(bat.x[1]), P(bat.y[0]), P(bat.y[1]), P(bat.f),
                       P(bat.insts), P(bat.state), P(bat.active_inst), P(bat.unit_off), P(bat.nact),
                       ctypes.byref(cfg), bat.multi, bat.stream_rows, bat.sgrid, s)
@@ -118,7 +122,15 @@ def roofline_phase(bat, reps, rule):
             bat._call("opy_tv_primal" + sfx, P(bat.x[0]), P(bat.x[1]), P(bat.y[0]), P(bat.f), P(bat.insts),
                       P(bat.state), P(bat.active_inst), P(bat.act_off), P(bat.nact), ctypes.byref(cfg), bat.grid, s)
 
-    out = {"grid": bat.sgrid if (bat.multi > 1 and bat._use_stream(cfg)) else bat.grid}
+    def blocks():
+        return bat.wgrid if bat._use_wide(cfg) else bat.sgrid if bat.multi > 1 and bat._use_stream(cfg) else bat.grid
+
+    tlen = bat.multi  # the steps of the launches below: the first K of the rule
+    if bat._use_wide(cfg):
+        table = torch.zeros(bat.B * bat.multi * 8, dtype=torch.float32, device="cuda")
+        bat._call("opy_tv_wide_steps", P(bat.insts), P(bat.state), P(bat.checks), bat.B, ctypes.byref(cfg), tlen,
+                  P(table), s)
+    out = {"grid": blocks()}
     if bat.passes == 2:
         names = ("dual", "primal")
     else:
@@ -133,7 +145,7 @@ def roofline_phase(bat, reps, rule):
         e1.record(stream)
         torch.cuda.synchronize()
         out[name] = e0.elapsed_time(e1) / reps
-    if names == ("multi",) and bat._use_stream(cfg) and bat.multi != 4:
+    if names == ("multi",) and (bat._use_wide(cfg) or bat._use_stream(cfg)) and bat.multi > 4:
         # the same kernel at 4 iterations per launch, where HBM rather than
         # instruction issue bounds it
         k0 = bat.multi
@@ -148,7 +160,7 @@ def roofline_phase(bat, reps, rule):
         e1.record(stream)
         torch.cuda.synchronize()
         out["multi_k4"] = e0.elapsed_time(e1) / reps
-        out["grid_k4"] = bat.sgrid
+        out["grid_k4"] = blocks()
         bat.set_multi(k0)
         bat.refresh_grid()
     # copy of a known size (2^28 floats = 1 GiB read + 1 GiB written): the counter scale
@@ -160,7 +172,7 @@ def roofline_phase(bat, reps, rule):
     return out
 
 
-def measured_traffic(npx, tile, passes, rule, multi, stream=False):
+def measured_traffic(npx, tile, passes, rule, multi, kind):
     """(HBM bytes per full-batch launch of the dominant kernel, where they come
     from): the committed counter runs (FETCH_SIZE and WRITE_SIZE, each scaled
     by what it reads for a copy of known size), when they were taken on this
@@ -168,7 +180,7 @@ def measured_traffic(npx, tile, passes, rule, multi, stream=False):
     if passes == 2:
         name = "tv_dual_kernel"
     elif multi > 1:
-        name = ("tv_stream_kernel_k%d" if stream else "tv_multi_kernel_k%d") % multi
+        name = "tv_%s_kernel_k%d" % (kind, multi)
     else:
         name = "tv_iter_kernel"
     name += "_accel" if rule == "accel" else ""
@@ -322,11 +334,12 @@ LIFT_OMEGA = 6.0  # primal weight of the batched lifting solve (1 = the referenc
 
 
 def lifting_kernels(bat, A, N, k, reps):
-    """Eager full-batch launches of the fused lifting passes and, for scale,
-    of the generic chain's per-pixel product on the matrix cores (r (N, k) ->
+    """Eager full-batch launches of the fused lifting iteration and, for scale,
+    of its two passes and the generic chain's per-pixel product on the matrix cores (r (N, k) ->
     z (N, 2k), the MatrixMultR of one instance), timed with HIP events on
-    their stream.  Algorithmic bytes of a fused iteration: the primal pass
-    reads U, r, p (2), z (2) and writes U, x_bar's U, r, x_bar's r: 10
+    their stream.  Algorithmic bytes: the one-pass iteration reads U, r, p (2),
+    z (2) and f and writes U, r, p (2), z (2): 12 planes of k values per pixel
+    and f; of the two passes, the primal one reads U, r, p (2), z (2) and writes U, x_bar's U, r, x_bar's r: 10
     planes of k values per pixel; the dual pass reads x_bar (2), p (2), z (2)
     and f and writes p (2), z (2): 10 planes plus f."""
     import torch
@@ -349,6 +362,11 @@ def lifting_kernels(bat, A, N, k, reps):
                                         Pt(bat.f), *ctl()), 10 * npl * es + npx * es),
         "matmul_r_mfma (one instance, generic chain)": (lambda: mm(r, z), N * 3 * k * 4),
     }
+    if bat._one_pass():
+        U1, p1, z1 = bat._other
+        cases["lift_iter"] = (lambda: bat._call("opy_lift_iter" + bat._sfx(), Pt(bat.U), Pt(U1), Pt(bat.r), Pt(bat.p),
+                                                Pt(p1), Pt(bat.z), Pt(z1), Pt(bat.f), *ctl()),
+                              12 * npl * es + npx * es)
     out = {}
     for name, (fn, nbytes) in cases.items():
         fn()
@@ -464,9 +482,9 @@ def lifting_main(args, emit=True):
                "sample": "oracle (float64 numpy/scipy, 1 thread): %d preconditioned iterations of one 512x512, "
                          "L=16 instance in %.1fs (step set-up included), scaled to the mean %d iterations per "
                          "instance of the GPU batch" % (n_it, dt, it0)}
-    prim, dual = kt["lift_primal"], kt["lift_dual"]
-    it_ms = prim["ms"] + dual["ms"]
-    it_bytes = prim["bytes"] + dual["bytes"]
+    passes = [kt["lift_iter"]] if "lift_iter" in kt else [kt["lift_primal"], kt["lift_dual"]]
+    it_ms = sum(q["ms"] for q in passes)
+    it_bytes = sum(q["bytes"] for q in passes)
     achieved = it_bytes / (it_ms * 1e-3) / 1e9
     line = {
         "metric": "solves/sec to rel PD-gap 1e-5: batched+warm-start vs plain PDHG; %HBM peak",
@@ -487,9 +505,10 @@ def lifting_main(args, emit=True):
                    "kernels": kt},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": None, "traffic_source": None,
-                     "kernel": "lift_primal_kernel<float,16> + lift_dual_kernel<float,16>: one iteration over the "
-                               "batch, %d B algorithmic (20 planes of k=%d FP32 values per pixel, and f)"
-                               % (it_bytes, k),
+                     "kernel": "%s: one iteration over the batch, %d B algorithmic (%d planes of k=%d FP32 values "
+                               "per pixel, and f)"
+                               % (("lift_iter_kernel<float,16>", it_bytes, 12, k) if len(passes) == 1 else
+                                  ("lift_primal_kernel<float,16> + lift_dual_kernel<float,16>", it_bytes, 20, k)),
                      "avg_ms": it_ms},
         "cpu_baseline": cpu,
     }
@@ -629,8 +648,10 @@ def main():
         log("batched (%s start, for comparison): %d/%d certified in %.2fs" % (other["start"], c, args.batch, dt))
 
     kt = roofline_phase(bat, args.reps, args.step_rule)
-    stream_used = bat.multi > 1 and bat._use_stream(bat._cfg(args.step_rule))
-    stream_rows = bat.stream_rows
+    bcfg = bat._cfg(args.step_rule)
+    kind = "wide" if bat._use_wide(bcfg) else "stream" if bat.multi > 1 and bat._use_stream(bcfg) else "multi"
+    unit_rows = {"wide": bat.wrows, "stream": bat.stream_rows}.get(kind)
+    lane_cols = 128 if kind == "wide" else 64
     variant = "adaptive" if args.step_rule == "adaptive" else "accelerated steps"
     k_launch = 1
     if bat.passes == 2:
@@ -639,10 +660,11 @@ def main():
     elif "multi" in kt:
         k_launch = bat.multi
         kname, kms, kbytes = "multi", kt["multi"], MULTI_BYTES_PER_PX
-        if stream_used:
-            kdesc = ("tv_stream_kernel<float,1,%d>, %s (%d iterations per launch, one wavefront per %d x %d unit, "
-                     "the iterations pipelined down its rows)" % (k_launch, variant, k_launch, 64 - 2 * k_launch,
-                                                                  stream_rows))
+        if unit_rows:
+            kdesc = ("%s, %s (%d iterations per launch, one wavefront per %d x %d unit, the iterations pipelined down "
+                     "its rows)" % ("tv_wide_kernel<%d>" % k_launch if kind == "wide" else
+                                    "tv_stream_kernel<float,1,%d>" % k_launch, variant, k_launch,
+                                    lane_cols - 2 * k_launch, unit_rows))
         else:
             kdesc = "tv_multi_kernel<float,1,%d,%d>, %s (%d iterations per launch on LDS-staged tiles)" % (
                 args.tile[1], k_launch, variant, k_launch)
@@ -682,7 +704,7 @@ def main():
                lift["roofline"]["achieved"]))
 
     from opymize_amd.solvers import tv as tvmod
-    traffic = measured_traffic(npx, args.tile, args.passes, args.step_rule, k_launch, stream=stream_used)
+    traffic = measured_traffic(npx, args.tile, args.passes, args.step_rule, k_launch, kind)
     line = {
         "metric": "solves/sec to rel PD-gap 1e-5: batched+warm-start vs plain PDHG; %HBM peak",
         "value": value, "unit": "solves/s", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
@@ -702,8 +724,8 @@ def main():
                     "median_per_instance": float(np.median(nrestarts))},
                    "other_start": other,
                    "tile": list(args.tile), "block_iters": args.block_iters, "iterations_per_launch": k_launch,
-                   "multi_kernel": ("stream" if stream_used else "tile") if k_launch > 1 else None,
-                   "stream_rows": stream_rows if stream_used else None,
+                   "multi_kernel": {"multi": "tile"}.get(kind, kind) if k_launch > 1 else None,
+                   "stream_rows": unit_rows if k_launch > 1 else None,
                    "certified": int(certified), "instances": int(args.steps * args.batch),
                    "iterations_median": float(np.median(iters)), "iterations_max": int(iters.max()),
                    "plain_single_instance_solves_per_sec": plain["value"] if plain else None,
@@ -725,21 +747,21 @@ def main():
         "cpu_baseline": cpu,
     }
     if "multi_k4" in kt:
-        # the same kernel at 4 iterations per launch (same bytes per launch):
-        # beyond 4 the launch is bound by instruction issue, not HBM, and it is
-        # the time per iteration the solve needs
+        # the same kernel at 4 iterations per launch (the same algorithmic bytes
+        # per launch): beyond 4 the launch is bound by instruction issue, not
+        # HBM, and it is the time per iteration the solve needs
         a4 = kbytes * npx / (kt["multi_k4"] * 1e-3) / 1e9
         line["roofline"]["note"] = ("%d iterations per launch: bound by instruction issue (VALU; SQ_INSTS_VALU in "
                                     "the committed profile of this kernel), %.3f ms per iteration, %.1f TB/s of "
                                     "single-iteration traffic (28 B/pixel per iteration); the same kernel at 4 per "
-                                    "launch is HBM-bound, see roofline_k4"
+                                    "launch moves more bytes per second, see roofline_k4"
                                     % (k_launch, kms / k_launch, achieved * k_launch / 1e3))
         line["roofline_k4"] = {"bound": "hbm", "achieved": a4, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                "frac": a4 / HBM_PEAK_GBS, "avg_ms": kt["multi_k4"],
                                "ms_per_iteration": kt["multi_k4"] / 4, "blocks_per_launch": kt["grid_k4"],
-                               "kernel": "the same streaming kernel with 4 iterations per launch (%d x %d units), "
-                                         "%d B/pixel algorithmic x %d pixels per launch"
-                                         % (56, stream_rows, kbytes, npx)}
+                               "kernel": "the same streaming kernel with 4 iterations per launch (strips of %d "
+                                         "columns), %d B/pixel algorithmic x %d pixels per launch"
+                                         % (lane_cols - 8, kbytes, npx)}
     print(json.dumps(line), flush=True)
 
 
