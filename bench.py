@@ -34,7 +34,7 @@ Printed next to it:
     --multi 1 or adaptive steps; the dual pass with --passes 2): algorithmic
     bytes of a full-batch launch over the average duration of eager
     full-batch launches, timed with HIP events on the launch stream; with
-    K > 4 also the same kernel at K = 4 (roofline_k4), where HBM rather than
+    K > 4 also the streaming kernel at K = 4 (roofline_k4), where HBM rather than
     instruction issue bounds it;
   * the CPU oracle (float64 numpy/scipy, one thread) on a bounded sample,
     and a pool of processes running it on as many instances at once.
@@ -161,6 +161,7 @@ def roofline_phase(bat, reps, rule):
         torch.cuda.synchronize()
         out["multi_k4"] = e0.elapsed_time(e1) / reps
         out["grid_k4"] = blocks()
+        out["grid_cols_k4"] = (128 if bat._use_wide(cfg) else 64) - 8
         bat.set_multi(k0)
         bat.refresh_grid()
     # copy of a known size (2^28 floats = 1 GiB read + 1 GiB written): the counter scale
@@ -753,15 +754,15 @@ def main():
         a4 = kbytes * npx / (kt["multi_k4"] * 1e-3) / 1e9
         line["roofline"]["note"] = ("%d iterations per launch: bound by instruction issue (VALU; SQ_INSTS_VALU in "
                                     "the committed profile of this kernel), %.3f ms per iteration, %.1f TB/s of "
-                                    "single-iteration traffic (28 B/pixel per iteration); the same kernel at 4 per "
+                                    "single-iteration traffic (28 B/pixel per iteration); the streaming kernel at 4 per "
                                     "launch moves more bytes per second, see roofline_k4"
                                     % (k_launch, kms / k_launch, achieved * k_launch / 1e3))
         line["roofline_k4"] = {"bound": "hbm", "achieved": a4, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                "frac": a4 / HBM_PEAK_GBS, "avg_ms": kt["multi_k4"],
                                "ms_per_iteration": kt["multi_k4"] / 4, "blocks_per_launch": kt["grid_k4"],
-                               "kernel": "the same streaming kernel with 4 iterations per launch (strips of %d "
+                               "kernel": "the streaming kernel with 4 iterations per launch (strips of %d "
                                          "columns), %d B/pixel algorithmic x %d pixels per launch"
-                                         % (lane_cols - 8, kbytes, npx)}
+                                         % (kt["grid_cols_k4"], kbytes, npx)}
     print(json.dumps(line), flush=True)
 
 
