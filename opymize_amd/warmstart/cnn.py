@@ -210,7 +210,7 @@ class ConvNet(object):
                   _hip.ptr(self.grads[l * self.per:(l + 1) * self.per]), s)
             if l > 0:
                 # dL/d(output of layer l - 1) through its ReLU: zero where that output is not positive
-                gn = bufs[l % 2]
+                gn = bufs[(l - 1) % 2]
                 _call("opy_conv3x3_bwd_data", _hip.ptr(g), _hip.ptr(gn), _hip.ptr(self._wb[l]), _hip.ptr(acts[l]),
                       N, H, W, self.grid, s)
                 g = gn

@@ -93,6 +93,32 @@ def test_network_loss_and_gradients_match_oracle(gpu):
         rel_close(gb, grads_ref[l][1], tol=1e-2)
 
 
+@pytest.mark.parametrize("layers", [1, 2, 4])
+def test_gradients_of_every_depth(gpu, layers):
+    """The backward pass hands its gradient from layer to layer through two
+    buffers at most: depths that need none, one and both of them (tolerances as
+    for the three-layer network above)."""
+    from opymize_amd.warmstart.cnn import ConvNet
+    rng = np.random.default_rng(8 + layers)
+    N, H, W = 1, 11, 35
+    net = ConvNet(layers=layers, n_in=2, n_out=3, seed=9)
+    x = np.zeros((N, H, W, 32), dtype=np.float32)
+    x[..., :2] = rng.standard_normal((N, H, W, 2))
+    tgt = np.zeros_like(x)
+    tgt[..., :3] = rng.standard_normal((N, H, W, 3))
+    params = [(net.W(l).cpu().numpy().reshape(9, 32, 32).astype(np.float64),
+               net.b(l).cpu().numpy().astype(np.float64)) for l in range(layers)]
+    xd, td = torch.as_tensor(x).cuda(), torch.as_tensor(tgt).cuda()
+    before = net.params.clone()
+    net.train_step(xd, td, lr=1e-3)
+    assert not torch.equal(net.params, before)
+    _, grads_ref = cnn.net_loss_grad(x, tgt, params, nc=3)
+    G = net.grads.cpu().numpy()
+    for l in range(layers):
+        rel_close(G[l * net.per:l * net.per + 9 * 1024].reshape(9, 32, 32), grads_ref[l][0], tol=1e-2)
+        rel_close(G[l * net.per + 9 * 1024:(l + 1) * net.per], grads_ref[l][1], tol=1e-2)
+
+
 def test_training_reduces_loss(gpu):
     """Fit a fixed smoothing target: loss must drop by 10x within 300 Adam steps."""
     from opymize_amd.warmstart.cnn import ConvNet
