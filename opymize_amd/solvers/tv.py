@@ -134,6 +134,9 @@ def _wide_strips(W, sw):
 # iterations per streaming launch from which blocks run without a graph (_captured)
 CAPTURE_BELOW = 4
 
+# rows per thread that the tile kernel of several iterations per launch is built for
+MULTI_ROWS = (2, 4, 6, 8)
+
 # rows per unit that the two-column kernel may take (wide_rows)
 WIDE_ROWS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 52, 57, 64, 69, 74, 80, 86, 94, 103, 114, 128,
              147, 171, 205, 256, 342, 512)
@@ -601,10 +604,20 @@ class TVBatch(object):
         return n
 
     def _iterations(self, n, cfg, adapt, params):
-        """n iterations starting from buffer self.cur (updates self.cur)."""
+        """n iterations starting from buffer self.cur (updates self.cur).  What a
+        block leaves over of the two-column kernel's launches goes to the tile
+        kernel: 700 iterations of one 64^2 image in blocks of 14 at 8 per launch
+        take 2.7 ms that way, 5.2 with single iterations for the rest."""
         k = self._launch_k(cfg) if not adapt else 1
-        if k > 1 and n >= k and self._use_wide(cfg):
-            n = self._wide_iterations(n, cfg, k)
+        if k > 1 and self._use_wide(cfg):
+            if n >= k:
+                n = self._wide_iterations(n, cfg, k)
+            k = 1
+            while n > 1 and self.rpt in MULTI_ROWS:
+                m = min(n, 4)
+                self._multi_launch(self.cur, cfg, m)
+                self.cur ^= 1
+                n -= m
         while k > 1 and n >= k:
             self._multi_launch(self.cur, cfg, k)
             self.cur ^= 1
@@ -645,8 +658,8 @@ class TVBatch(object):
             g.replay()
             self.cur = end
 
-    def _captured(self, cfg, adapt):
-        """Whether blocks of launches are worth a captured graph.  A capture
+    def _captured(self, cfg, adapt, n):
+        """Whether blocks of n iterations are worth a captured graph.  A capture
         costs 0.3 to 0.4 ms and the replay after each check's read starts 10 us
         later than plain launches, which single iterations (a few us each) earn
         back and the streaming kernels' launches, longer than the host takes
@@ -654,8 +667,18 @@ class TVBatch(object):
         captured against plain, one image of 64^2 takes 2.9 / 18.4 against 2.6 /
         25.3 ms at 2 iterations per launch, 2.5 / 17.7 against 1.8 / 16.1 at 4 and
         2.7 / 20.8 against 2.1 / 19.1 at 8, one of 1024^2 3.3 / 26.7 against 2.7 /
-        24.9 at 8."""
-        return adapt or self._launch_k(cfg) < CAPTURE_BELOW or not (self._use_wide(cfg) or self._use_stream(cfg))
+        24.9 at 8.  A block shorter than one such launch is captured (blocks of 6
+        at 8 per launch, 64^2: 2.2 ms per 300 iterations, 4.6 plain as single
+        launches), and so is one whose rest is left to single iterations; on tiles
+        the rest takes at most two launches (blocks of 14, 700 iterations: 2.7 ms
+        plain, 3.6 captured)."""
+        if adapt:
+            return True
+        k = self._launch_k(cfg)
+        wide = self._use_wide(cfg)
+        if k < CAPTURE_BELOW or n < k or not (wide or self._use_stream(cfg)):
+            return True
+        return n % k > 1 and not (wide and self.rpt in MULTI_ROWS)
 
     def _to_buffer0(self):
         """Bring each instance's iterate to buffer 0 (the start and result
@@ -793,7 +816,7 @@ class TVBatch(object):
             self._wide_alloc()  # before any block is captured
 
         def graphs():
-            return use_graph and self._captured(cfg, adapt)
+            return use_graph and self._captured(cfg, adapt, block_iters)
         # captured blocks per (launch grid, buffer holding the iterate at the start)
         g_it, g_ck = {"warm": False}, {"warm": False}
         done_iters, nblk = 0, 0

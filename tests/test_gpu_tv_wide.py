@@ -42,6 +42,35 @@ def test_wide_equals_single_launches(gpu, monkeypatch, multi, rows, steps):
     assert gaps == gaps1
 
 
+@pytest.mark.parametrize("multi,block", [(8, 6), (8, 7), (8, 13), (8, 15), (4, 7), (5, 9), (3, 5), (8, 2)])
+def test_rest_of_a_block_takes_few_launches(gpu, monkeypatch, multi, block):
+    """What a block leaves over of whole launches (all of it where it is
+    shorter than one) runs on tiles of up to four iterations, at most one
+    iteration by itself; the iterates of single launches, captured or not."""
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 3 + i) for i, (H, W) in enumerate(SHAPES)]
+    data = ["l1" if i % 3 == 1 else "l2" for i in range(len(SHAPES))]
+    out = []
+    for m, graph in ((multi, False), (multi, True), (1, True)):
+        bat = tv.TVBatch(imgs, 3.0, data, multi=m)
+        names = []
+        call = bat._call
+        monkeypatch.setattr(bat, "_call", lambda name, *a: (names.append(name), call(name, *a))[1])
+        res = bat.solve(steps="accel", step_bound=0.124, max_iters=4 * block, block_iters=block, tol=1e-30,
+                        use_graph=graph)
+        out.append((bat.solution(), [r["gap"] for r in res]))
+        if m > 1 and not graph:
+            rest = block % multi
+            count = [names.count("opy_tv_" + k) for k in ("wide_f32", "multi_f32", "iter_f32")]
+            assert count == [4 * (block // multi), 4 * ((rest + 2) // 4), 4 * (rest % 4 == 1)]
+        if m == 8:
+            assert bat._captured(bat._cfg("accel"), False, block) == (block < 8)
+    for (xs, ys), gaps in out[:2]:
+        for a, b in zip(xs + ys, out[2][0][0] + out[2][0][1]):
+            np.testing.assert_array_equal(a, b)
+        assert gaps == out[2][1]
+
+
 def test_kernel_may_change_between_blocks(gpu, monkeypatch):
     """Fewer than 6 iterations per launch: one column per lane while the batch
     is large, two from the check on at which enough instances stopped; captured
