@@ -372,10 +372,19 @@ inline bool use_3d_forward(const Grid& g) {
                          g.h[1], g.h[2], add);                                                              \
   } while (0)
 
-// The 2-D kernels serve forward 2-D grids whose indices fit 32 bits and whose
-// rows fit the grid's second dimension.
+// The 2-D kernels serve 2-D grids whose indices fit 32 bits and whose rows fit
+// the grid's second dimension.
 inline bool use_2d(const Grid& g) {
   return g.ndims == 2 && g.dims[0] >= 1 && g.dims[0] <= 65535 && g.npoints * g.nchan * 2 < (int64_t(1) << 31);
+}
+
+// The centered ones give every row a block of its own, 0.46 ns each however
+// short the row is, where the n-D kernels take 0.011 ns per value: many short
+// rows stay on those.  A gradient and its adjoint, n-D / 2-D, us: 65535 rows of
+// 1 value 6.5 / 60, of 16 28 / 62, of 32 51 / 60, of 64 93 / 61; 20000 rows of 16
+// 13 / 21, of 64 33 / 24; 5000 rows of 2 8.6 / 8.0; 1000 rows of 8 8.6 / 4.5.
+inline bool use_2d_centered(const Grid& g) {
+  return use_2d(g) && (g.dims[0] <= 5000 || g.dims[1] * g.nchan >= 40);
 }
 
 // vec: the field (the gradient's output, the divergence's input) is aligned for 2-vector accesses
@@ -626,7 +635,7 @@ int grad_impl(const T* x, T* y, const opy_grid_t* gd, const double* w, int schem
   if (int rc = make_grid(gd, &g)) return rc;
   if (!x || !y) return fail(kInvalid, "gradient: null pointer");
   const int64_t n = g.npoints * g.nchan;
-  if (scheme == OPY_SCHEME_CENTERED && use_2d(g)) {
+  if (scheme == OPY_SCHEME_CENTERED && use_2d_centered(g)) {
     if (n > 0) OPY_LAUNCH_2F(grad2c_kernel, T, x, y, g, w, add, as_stream(s),
                              reinterpret_cast<uintptr_t>(y) % (2 * sizeof(T)) == 0);
   } else if (scheme == OPY_SCHEME_CENTERED)
@@ -649,7 +658,7 @@ int div_impl(const T* p, T* x, const opy_grid_t* gd, const double* w, int scheme
   if (int rc = make_grid(gd, &g)) return rc;
   if (!x || !p) return fail(kInvalid, "divergence: null pointer");
   const int64_t n = g.npoints * g.nchan;
-  if (scheme == OPY_SCHEME_CENTERED && use_2d(g)) {
+  if (scheme == OPY_SCHEME_CENTERED && use_2d_centered(g)) {
     if (n > 0) OPY_LAUNCH_2F(div2c_kernel, T, p, x, g, w, add, as_stream(s),
                              reinterpret_cast<uintptr_t>(p) % (2 * sizeof(T)) == 0);
   } else if (scheme == OPY_SCHEME_CENTERED)

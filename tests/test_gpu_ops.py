@@ -440,6 +440,58 @@ def test_centered_2d_at_edges(gpu, dims, C):
             assert np.abs(out.cpu().numpy() - ref).max() <= 1e-13 * max(1.0, np.abs(ref).max())
 
 
+@pytest.mark.parametrize("dims,C", [((5000, 3), 1), ((5001, 3), 1), ((5001, 39), 1), ((5001, 40), 1), ((5001, 13), 3),
+                                    ((5001, 14), 3)])
+def test_centered_routes_agree(gpu, dims, C):
+    """Either side of the line between the 2-D and the n-D kernels of the
+    centered scheme: the values of the sparse matrix (FP64, as above)."""
+    import torch
+    from opymize_amd.linear import GradientOp
+    from oracle import ops
+    rng = np.random.default_rng(dims[0] + dims[1] + C)
+    h, w = (0.5, 2.0), np.arange(1, C + 1) * 0.75
+    A = GradientOp(dims, C, scheme="centered", imageh=h, weights=w)
+    M = ops.grad_matrix(dims, C, h=np.array(h), w=w, scheme="centered")
+    x, y = rng.standard_normal(A.x.size), rng.standard_normal(A.y.size)
+    for op, mat, a, b in ((A, M, x, y), (A.adjoint, M.T, y, x)):
+        out = torch.as_tensor(b).cuda()
+        op(torch.as_tensor(a).cuda(), out)
+        ref = mat @ a
+        assert np.abs(out.cpu().numpy() - ref).max() <= 1e-13 * max(1.0, np.abs(ref).max())
+
+
+def test_centered_tall_grids_cost_what_their_points_do(gpu):
+    """65535 rows of one value, captured 20 times (no host time): not many
+    times what 256^2 takes (a block per row took 15 times as long)."""
+    import torch
+    from opymize_amd.linear import GradientOp
+    took = []
+    for dims in ((256, 256), (65535, 1)):
+        A = GradientOp(dims, 1, scheme="centered")
+        x, z = (torch.ones(A.x.size, device="cuda") for _ in range(2))
+        y = torch.zeros(A.y.size, device="cuda")
+
+        def pair():
+            A(x, y)
+            A.adjoint(y, z)
+        pair()
+        torch.cuda.synchronize()
+        g, s = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.graph(g, stream=s):
+            for _ in range(20):
+                pair()
+        best = float("inf")
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            g.replay()
+            b.record()
+            torch.cuda.synchronize()
+            best = min(best, a.elapsed_time(b))
+        took.append(best)
+    assert took[1] < 4 * took[0], took
+
+
 @pytest.mark.parametrize("n,m", [(1, 2), (257, 512), (300000, 600001)])
 def test_residuals_in_one_call_equal_the_separate_ones(gpu, n, m):
     """opy_pdhg_residuals against two opy_pdhg_residual2 calls and
