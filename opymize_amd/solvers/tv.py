@@ -269,6 +269,16 @@ class TVBatch(object):
         self._restart = None  # (beta, min_iters, tau0, sigma0) while a solve restarts its schedule
 
     # -- layout --------------------------------------------------------------
+    @property
+    def shapes(self):
+        """(H, W) of every instance."""
+        return self._shapes
+
+    @shapes.setter
+    def shapes(self, shapes):
+        self._shapes = list(shapes)
+        self._most_pixels = max(H * W for (H, W) in self._shapes)
+
     def set_multi(self, k):
         if not 1 <= int(k) <= 8:
             raise ValueError("multi must be 1 to 8 iterations per launch")
@@ -292,11 +302,14 @@ class TVBatch(object):
         if self.multi < 2:
             self.total_units = 0
             return
+        self._wide_strips = _wide_strips(self._W, WIDE_COLS - 2 * self.multi)
+        self._wide_work = self._wide_strips * self._H
         self._wide_sized = None
         self._size_wide(np.arange(self.B))
         sw, rows = 64 - 2 * self.multi, self.stream_rows
         self._strips = np.array([_stream_strips(W, sw) for (H, W) in self.shapes], dtype=np.int64)
-        self.total_units = int(np.sum(self._strips * -(-self._H // rows)))
+        self._units = self._strips * -(-self._H // rows)
+        self.total_units = int(self._units.sum())
         if self._grid_override is None:
             self.sgrid = self._stream_grid(self.total_units)
         else:
@@ -318,15 +331,15 @@ class TVBatch(object):
         running units return at once."""
         if self.C != 1 or self.dtype != torch.float32:
             return False
-        strips = _wide_strips(self._W, WIDE_COLS - 2 * self.multi)
-        work = strips * self._H
+        work = self._wide_work
         share = -(-16 * int(work[running].sum()) // int(work.sum())) if len(running) else 0
         if share == self._wide_sized or share == 0:
             return False
         self._wide_sized = share
         was = self.wrows
-        self.wrows = wide_rows(self._H[running], strips[running], self.multi, self._simds)
-        units = int(np.sum(strips[running] * -(-self._H[running] // self.wrows)))
+        H, strips = self._H[running], self._wide_strips[running]
+        self.wrows = wide_rows(H, strips, self.multi, self._simds)
+        units = int(np.sum(strips * -(-H // self.wrows)))
         self.wgrid = -(-max(units, 1) // 8) * 8
         return self.wrows != was
 
@@ -374,7 +387,7 @@ class TVBatch(object):
         """Every instance's y block (2 C values per pixel) is below 4 GiB, the
         reach of the streaming kernel's 32-bit offsets."""
         esize = 4 if self.dtype == torch.float32 else 8
-        return max(H * W for (H, W) in self.shapes) * 2 * self.C * esize < (1 << 32)
+        return self._most_pixels * 2 * self.C * esize < (1 << 32)
 
     def _launch_k(self, cfg):
         """Iterations per K-iteration launch: multi, or at most 4 on the tile
@@ -448,7 +461,7 @@ class TVBatch(object):
         self._running_now = now
         self.grid = self._launch_grid(int(run[self.B + 1 + nrun]))
         if self.multi > 1:
-            units = int(np.sum(self._strips[running] * -(-self._H[running] // self.stream_rows)))
+            units = int(self._units[running].sum())
             if self._grid_override is None:
                 self.sgrid = self._stream_grid(units)
             self._stream_now = units >= self.stream_min_units

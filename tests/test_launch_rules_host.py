@@ -2,6 +2,7 @@
 streaming kernel, rows per thread of the single-pass tile kernel."""
 import numpy as np
 import pytest
+import torch
 
 from opymize_amd.solvers import autotune, tv
 
@@ -19,6 +20,28 @@ def test_wide_rows_fill_the_chip(shapes, k):
         assert rows == 1
     else:
         assert units >= 512
+
+
+def test_kernel_choice_does_not_walk_the_batch():
+    """The choice is made several times per block: its cost must not grow with
+    the number of instances."""
+    class Shapes(list):
+        closed = False
+
+        def __iter__(self):
+            assert not self.closed, "walked the instances"
+            return list.__iter__(self)
+
+    bat = object.__new__(tv.TVBatch)
+    bat.C, bat.dtype, bat.multi, bat.multi_kernel, bat._wide_now, bat._stream_now = 1, torch.float32, 8, "auto", True, True
+    cfg = tv.TVCfg()
+    cfg.steps = tv.STEP_MODES["accel"]
+    shapes = Shapes([(64, 64), (30, 500)])
+    bat.shapes = shapes
+    bat._shapes, shapes.closed = shapes, True
+    assert bat._use_wide(cfg) and bat._use_stream(cfg) and bat._launch_k(cfg) == 8
+    bat.shapes = [(64, 64), (23171, 23171)]  # 2 x 4 B x 23171^2 > 2^32
+    assert not bat._use_wide(cfg)
 
 
 @pytest.mark.parametrize("C", [1, 2, 3, 4])
