@@ -62,6 +62,7 @@ CHECK_DOUBLES = ctypes.sizeof(TVCheck) // 8
 RESTART_DOUBLES = ctypes.sizeof(TVRestart) // 8
 STATE_DOUBLES = _hip.ADAPT_STATE_DOUBLES
 STREAM_MIN_UNITS = 4096
+WIDE_UNITS = {2: 2048, 3: 4096, 4: 4096, 5: 8192}  # iterations per launch: see _use_wide
 WIDE_COLS = 128   # columns of a strip of the two-column streaming kernel
 WIDE_TABLE = 64   # iterations whose step coefficients it takes from one table
 assert ctypes.sizeof(TVInst) == 48 and ctypes.sizeof(TVCfg) == 64 and ctypes.sizeof(TVCheck) == 72
@@ -371,12 +372,16 @@ class TVBatch(object):
 
     def _use_wide(self, cfg):
         """Whether the next K-iteration launches run the two-column streaming
-        kernel.  Below 6 iterations per launch a batch with more than 8192 of
-        the one-column kernel's units is left to that one: both wait for HBM
-        there, and it has twice the wavefronts to wait with (240 iterations of
-        128 images of 1024^2 with 2, 4, 5 per launch: one column 114, 55.2,
-        47.9 ms, two columns 119, 57.9, 48.6; with 6 40.6 against 39.2; of 32
-        images 27.0, 13.1, 11.5 against 25.6, 12.6, 11.2)."""
+        kernel.  Below 6 iterations per launch a batch of many of the one-column
+        kernel's units (WIDE_UNITS) is left to the other kernels: HBM bounds
+        them all there, and those have more wavefronts to wait with.  240
+        iterations, ms, on tiles / in one column / in two: 96 images of sides 64
+        to 1024 (4100 to 4400 units) 23.0 / 23.5 / 26.1 with 2 per launch, - / 17.0 /
+        17.9 with 3, - / 12.6 / 13.6 with 4, - / 11.1 / 11.0 with 5; 128 of 1024^2
+        - / 114 / 119 with 2, - / 55.2 / 57.9 with 4, - / 47.9 / 48.6 with 5 and
+        - / 40.6 / 39.2 with 6; 32 of 1024^2 (4600 units) 25.0 / 27.4 / 26.3 with
+        2, - / 13.8 / 13.2 with 4; 16 of 1024^2 (2300) 13.5 / - / 14.4 with 2, 11.3 /
+        - / 10.6 with 3; 6 of 1024^2 (860) 6.1 / - / 5.1 with 2."""
         return self._wide_fits(cfg) and self._wide_now
 
     def _wide_fits(self, cfg):
@@ -465,7 +470,7 @@ class TVBatch(object):
             if self._grid_override is None:
                 self.sgrid = self._stream_grid(units)
             self._stream_now = units >= self.stream_min_units
-            self._wide_now = self.multi >= 6 or units < 2 * STREAM_MIN_UNITS
+            self._wide_now = units < WIDE_UNITS.get(self.multi, units + 1)
             if self._size_wide(running):
                 self._stream_units()
         return nrun

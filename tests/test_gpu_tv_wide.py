@@ -76,7 +76,7 @@ def test_kernel_may_change_between_blocks(gpu, monkeypatch):
     is large, two from the check on at which enough instances stopped; captured
     blocks and the iterates of single launches, bit for bit."""
     from opymize_amd.solvers import tv
-    monkeypatch.setattr(tv, "STREAM_MIN_UNITS", 3)
+    monkeypatch.setattr(tv, "WIDE_UNITS", {3: 6})
     imgs = [rects(H, W, 30 + i) for i, (H, W) in enumerate([(60, 140), (33, 250), (90, 64), (20, 300)])]
     out = []
     for multi in (3, 1):
@@ -90,6 +90,23 @@ def test_kernel_may_change_between_blocks(gpu, monkeypatch):
     assert out[0][0] == out[1][0]
     for a, b in zip(out[0][1][0] + out[0][1][1], out[1][1][0] + out[1][1][1]):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("multi,side,n,wide", [(2, 1024, 14, True), (2, 1024, 16, False), (4, 512, 60, True),
+                                               (4, 512, 110, False), (5, 512, 110, True), (5, 512, 210, False),
+                                               (6, 512, 210, True)])
+def test_large_batches_below_six_per_launch(gpu, multi, side, n, wide):
+    """Which kernel a batch takes either side of WIDE_UNITS."""
+    import torch
+    from opymize_amd.solvers import tv
+    bat = tv.TVBatch([np.zeros((side, side))] * n, 3.0, "l2", multi=multi)
+    bat.solve(steps="accel", step_bound=0.124, max_iters=multi, block_iters=multi, tol=0.0)
+    bat.checks.zero_()  # all running, whatever the check of a zero image says
+    bat._compact(0)
+    assert bat.refresh_grid() == n
+    assert bat._use_wide(bat._cfg("accel")) == wide
+    del bat
+    torch.cuda.empty_cache()
 
 
 def test_wide_units_follow_the_running_instances(gpu):
