@@ -446,7 +446,8 @@ int opy_tv_stream_units(const opy_tv_inst_t* insts, const int32_t* active_inst, 
  * units of 128-2k columns by `rows` rows (strips(W) = the smaller of ceil(W / sw), sw = 128 - 2k, and of the
  * layout whose first and last strips carry no halo beyond the image edge: 1 for W <= 128, else
  * ceil((W - 128) / sw) + 1).  The launch runs the iterations it0 .. it0+k-1 of the n whose coefficients
- * opy_tv_wide_steps wrote to `table`; `grid` > 0 wavefronts (blocks of 64) walk the units.
+ * opy_tv_wide_steps wrote to `table`; `grid` > 0 wavefronts (blocks of 64), with 0 as many as are
+ * resident at once, walk the units.
  *   opy_tv_wide_steps: the coefficients of the next n iterations of every running instance's schedule (SCALAR or
  *     ACCEL steps) to table (B x n x 8 floats, 32-byte aligned) and, with ACCEL, its state advanced by n;
  *   opy_tv_wide_units: the exclusive prefix of the running instances' units of these strips (wide_off), and of

@@ -527,7 +527,7 @@ __host__ __device__ inline int stream_strips(int W, int sw) {
 
 // Blocks of `kernel` resident at once on the current device (occupancy x
 // CUs), cached per kernel and device: the persistent loops need no more.
-int resident_blocks(const void* kernel) {
+int resident_blocks(const void* kernel, int threads) {
   static std::mutex mu;
   static std::map<std::pair<const void*, int>, int> cache;
   int dev = 0;
@@ -537,7 +537,7 @@ int resident_blocks(const void* kernel) {
   const auto it = cache.find(key);
   if (it != cache.end()) return it->second;
   int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kTB, 0) != hipSuccess || per_cu < 1) per_cu = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0) != hipSuccess || per_cu < 1) per_cu = 1;
   if (dev < 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1)
     cus = 256;
   const int g = per_cu * cus;
@@ -546,7 +546,9 @@ int resident_blocks(const void* kernel) {
 }
 
 // grid > 0: as given; grid == 0: the resident block count of the kernel
-inline int launch_grid(const void* kernel, int grid) { return grid > 0 ? grid : resident_blocks(kernel); }
+inline int launch_grid(const void* kernel, int grid, int threads = kTB) {
+  return grid > 0 ? grid : resident_blocks(kernel, threads);
+}
 
 int check_cfg(const opy_tv_cfg_t* c) {
   if (!c) return fail(kInvalid, "tv: null config");

@@ -452,15 +452,15 @@ OPY_API int opy_tv_wide_f32(const float* xi, float* xo, const float* yi, float* 
                             int grid, void* s) {
   if (k < 2 || k > kWideMaxK) return fail(kInvalid, "tv_wide: k = %d not in [2, %d]", k, kWideMaxK);
   if (rows < 1 || rows > kWideMaxRows) return fail(kInvalid, "tv_wide: rows = %d not in [1, %d]", rows, kWideMaxRows);
-  if (!xi || !xo || !yi || !yo || !f || !insts || !table || !active_inst || !unit_off || !nact || grid < 1)
-    return fail(kInvalid, "tv_wide: null pointer or grid < 1");
+  if (!xi || !xo || !yi || !yo || !f || !insts || !table || !active_inst || !unit_off || !nact || grid < 0)
+    return fail(kInvalid, "tv_wide: null pointer or negative grid");
   if (n < 1 || it0 < 0 || it0 + k > n) return fail(kInvalid, "tv_wide: iterations %d..%d outside the table of %d", it0, it0 + k, n);
   if ((reinterpret_cast<uintptr_t>(table) & 31) != 0) return fail(kInvalid, "tv_wide: the table must be 32-byte aligned");
   if (xi == xo || yi == yo) return fail(kInvalid, "tv_wide: ping-pong buffers must differ");
   const WideStep* tab = reinterpret_cast<const WideStep*>(table);
-#define OPY_W(KK)                                                                                                    \
-  hipLaunchKernelGGL((tv_wide_kernel<KK>), dim3(grid), dim3(64), 0, as_stream(s), xi, xo, yi, yo, f, insts, tab, n, \
-                     it0, active_inst, unit_off, nact, rows)
+#define OPY_W(KK)                                                                                              \
+  hipLaunchKernelGGL((tv_wide_kernel<KK>), dim3(launch_grid(KF(tv_wide_kernel<KK>), grid, 64)), dim3(64), 0,    \
+                     as_stream(s), xi, xo, yi, yo, f, insts, tab, n, it0, active_inst, unit_off, nact, rows)
   switch (k) {
     case 2: OPY_W(2); break;
     case 3: OPY_W(3); break;

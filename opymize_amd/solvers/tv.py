@@ -341,7 +341,10 @@ class TVBatch(object):
         H, strips = self._H[running], self._wide_strips[running]
         self.wrows = wide_rows(H, strips, self.multi, self._simds)
         units = int(np.sum(strips * -(-H // self.wrows)))
-        self.wgrid = -(-max(units, 1) // 8) * 8
+        if self._grid_override is None:
+            self.wgrid = -(-max(units, 1) // 8) * 8
+        else:
+            self.wgrid = int(self._grid_override)
         return self.wrows != was
 
     def _stream_grid(self, units):

@@ -263,7 +263,8 @@ def test_launch_shapes_give_the_same_iterates(gpu, multi, rpt):
     lams = [2.0, 7.5, 1.0, 15.0, 4.0, 3.3]
     out = {}
     for grid in (None, 0, 7):
-        bat = TVBatch(imgs, lams, "l2", precision="float", tile=(64, rpt), grid=grid, multi=multi)
+        bat = TVBatch(imgs, lams, "l2", precision="float", tile=(64, rpt), grid=grid, multi=multi,
+                      multi_kernel="tile")
         if grid == 0:
             assert bat.grid == 0
         res = bat.solve(steps="accel", step_bound=0.124, max_iters=48, block_iters=24, tol=1e-30)

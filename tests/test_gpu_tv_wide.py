@@ -71,6 +71,29 @@ def test_rest_of_a_block_takes_few_launches(gpu, monkeypatch, multi, block):
         assert gaps == out[2][1]
 
 
+@pytest.mark.parametrize("multi", [3, 8])
+def test_wide_launch_shapes(gpu, multi):
+    """A block per unit, as many as are resident at once and seven, each of
+    which walks many units: the same iterates and gaps, bit for bit, after every
+    number of launches a check sees."""
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 3 + i) for i, (H, W) in enumerate(SHAPES)]
+    data = ["l1" if i % 3 == 1 else "l2" for i in range(len(SHAPES))]
+    out = {}
+    for grid in (None, 0, 7):
+        bat = tv.TVBatch(imgs, 3.0, data, multi=multi, grid=grid)
+        assert bat.wgrid == (grid if grid is not None else bat.wgrid)
+        res = bat.solve(steps="accel", step_bound=0.124, max_iters=72, block_iters=24, tol=1e-30)
+        assert bat._use_wide(bat._cfg("accel"))
+        units = int(bat.wide_off.cpu()[-1])
+        assert units > 100 and bat.wgrid == (-(-units // 8) * 8 if grid is None else grid)
+        out[grid] = (bat.solution(), [r["gap"] for r in res])
+    for g in (0, 7):
+        for a, b in zip(out[None][0][0] + out[None][0][1], out[g][0][0] + out[g][0][1]):
+            np.testing.assert_array_equal(a, b)
+        assert out[None][1] == out[g][1]
+
+
 def test_kernel_may_change_between_blocks(gpu, monkeypatch):
     """Fewer than 6 iterations per launch: one column per lane while the batch
     is large, two from the check on at which enough instances stopped; captured
