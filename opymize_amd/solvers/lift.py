@@ -131,14 +131,6 @@ class LiftBatch(object):
         self.r = torch.zeros(offk, dtype=dt, device="cuda")
         self.p = torch.zeros(2 * offk, dtype=dt, device="cuda")
         self.z = torch.zeros(2 * offk, dtype=dt, device="cuda")
-        # the one-pass iteration's second buffers of U, p and z; between its iterations they hold
-        # nothing, and the two-pass iteration keeps x_bar there
-        try:
-            self._other = tuple(torch.zeros_like(t) for t in (self.U, self.p, self.z))
-            self.Ub, self.rb = self._other[0], self._other[1][:offk]
-        except torch.cuda.OutOfMemoryError:  # a batch that only the two passes' buffers fit beside
-            self._other = None
-            self.Ub, self.rb = (torch.zeros(offk, dtype=dt, device="cuda") for _ in range(2))
         self.partials = torch.zeros(PARTIALS_PER_TILE * max(t0, 1), dtype=torch.float64, device="cuda")
         self.checks = torch.zeros(self.B * CHECK_DOUBLES, dtype=torch.float64, device="cuda")
         self.active_inst = torch.zeros(self.B, dtype=torch.int32, device="cuda")
@@ -146,6 +138,25 @@ class LiftBatch(object):
         self.nact = torch.zeros(1, dtype=torch.int32, device="cuda")
         self.iter_counter = torch.zeros(1, dtype=torch.int64, device="cuda")
         self.grid = max(1, t0)
+        # the one-pass iteration's second buffers of U, p and z (5 planes a piece beside the 6 of the
+        # state); between its iterations they hold nothing, and the two-pass iteration keeps x_bar
+        # there.  A batch that the two passes serve, or that would leave less memory free than these
+        # buffers take, gets x_bar's 2 planes alone.
+        self._other = None
+        if self._one_pass_serves() and self._room_for(5 * offk * self.U.element_size()):
+            try:
+                self._other = tuple(torch.zeros_like(t) for t in (self.U, self.p, self.z))
+                self.Ub, self.rb = self._other[0], self._other[1][:offk]
+            except torch.cuda.OutOfMemoryError:
+                pass
+        if self._other is None:
+            self.Ub, self.rb = (torch.zeros(offk, dtype=dt, device="cuda") for _ in range(2))
+
+    @staticmethod
+    def _room_for(nbytes):
+        """Whether nbytes can be taken and as much again stays free."""
+        cached = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
+        return 2 * nbytes <= torch.cuda.mem_get_info()[0] + cached
 
     # -- kernels ---------------------------------------------------------------
     def _sfx(self):
@@ -157,18 +168,21 @@ class LiftBatch(object):
         if rc != 0:
             raise _hip.HipError("%s failed: %s" % (name, lib.opy_last_error().decode()))
 
-    def _one_pass(self):
-        """Whether iterations run in pairs of the one-pass kernel: up to 24
-        pieces (FP64: 16), and beyond where every instance has that many.  Its
-        LDS holds the largest piece count of the batch for every tile, so with
-        more than 24 two blocks fit a CU and a batch of mixed counts is faster
-        in two passes (3 to 30 pieces 157 against 171 us per iteration, 3 to 23
-        pieces 127 against 105, 32 pieces throughout 186 against 163)."""
-        if self._other is None:
-            return False
+    def _one_pass_serves(self):
+        """Whether the one-pass kernel is the faster one for this batch: up to
+        24 pieces (FP64: 16), and beyond where every instance has more than 24.
+        Its registers and LDS are sized for the largest piece count of the batch
+        in every tile (FP32 blocks per CU by LDS: 8 up to 8 pieces, 4 up to 16, 2
+        beyond); the lines are where the times cross (us per iteration in one
+        and in two passes: 3 to 23 pieces 105 and 127, 3 to 30 pieces 171 and
+        157, 32 pieces throughout 163 and 186)."""
         if self.dtype != torch.float32:
             return self.kmax <= 16
         return self.kmax <= 24 or min(self.K) > 24
+
+    def _one_pass(self):
+        """Whether iterations run in pairs of the one-pass kernel."""
+        return self._other is not None
 
     def _iterations(self, n):
         """n iterations from and to the buffers U, r, p, z: pairs through the

@@ -176,3 +176,39 @@ def test_one_pass_iteration_equals_two_passes(gpu, precision, Ls):
     tol = 1e-12 if precision == "double" else 2e-5
     for a, b in zip(*out):
         assert np.abs(b).max() > 0 and np.abs(a - b).max() <= tol * max(1.0, np.abs(b).max())
+
+
+def test_second_buffers_only_where_they_serve(gpu, monkeypatch):
+    """5 planes for the one-pass iteration where it serves the batch and they
+    leave as much memory free, else x_bar's 2; the oracle's iterates either way
+    (FP64 1e-9) and the same values from both forms (1e-12 of the largest)."""
+    import torch
+    from opymize_amd.solvers.lift import LiftBatch
+    rng = np.random.default_rng(4)
+    img = [np.clip(0.5 + 0.2 * rng.standard_normal((13, 70)), 0, 1)]
+
+    def planes(lb):
+        bufs = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes()
+                for t in (lb.U, lb.r, lb.p, lb.z, lb.Ub, lb.rb) + (lb._other or ())}
+        return sum(bufs.values()) / (lb.n_planes * lb.U.element_size())
+
+    for L, precision, n in ((17, "double", 11), (18, "double", 8), (25, "float", 11), ([5, 30], "float", 8),
+                            ([28, 33], "float", 11)):
+        lb = LiftBatch(img * np.size(L), L, 0.2, precision=precision)
+        assert planes(lb) == n and (lb._other is not None) == (n == 11), (L, precision)
+    xs = []
+    for free in (None, 0):
+        if free is not None:
+            torch.cuda.empty_cache()
+            monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (free, 1 << 38))
+            monkeypatch.setattr(torch.cuda, "memory_reserved", torch.cuda.memory_allocated)
+        lb = LiftBatch(img, 9, 0.2, precision="double")
+        assert planes(lb) == (11 if free is None else 8)
+        lb.solve(max_iters=31, block_iters=31, check_every=1, tol=1e-30)
+        x, y = lb.solution()
+        xs.append(np.concatenate([x[0], y[0]]))
+    assert np.abs(xs[0] - xs[1]).max() <= 1e-12 * np.abs(xs[0]).max()
+    prob, _ = olf.problem(img[0], 9, 0.2)
+    xo, yo, _, _ = opd.solve(prob, steps="precond", term_maxiter=31, granularity=31, term_pd_gap=1e-30)
+    ref = np.concatenate([np.ravel(xo), np.ravel(yo)])
+    assert np.abs(xs[0] - ref).max() < 1e-9 * max(1.0, np.abs(ref).max())
