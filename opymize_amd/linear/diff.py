@@ -26,7 +26,8 @@ class _DiffBase(LinOp):
 
     def _grid(self):
         """The grid description, built again only when an attribute it is made of has changed."""
-        key = (tuple(self.imagedims), self.nchannels, self.imageh.tobytes())
+        h = self.imageh
+        key = (tuple(self.imagedims), self.nchannels, h.tobytes() if type(h) is np.ndarray else tuple(h))
         if self._grid_of[0] != key:
             self._grid_of = (key, _hip.make_grid(self.imagedims, self.nchannels, self.imageh))
         return self._grid_of[1]
