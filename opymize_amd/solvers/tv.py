@@ -151,7 +151,8 @@ def wide_rows(H, strips, k, simds):
     unit of r rows walks r + 2k of them, so few tall units are cheap; but a
     SIMD runs two units at once, in 1.54 of the time units that one alone
     takes 0.95 of, and those left over when the others have ended leave most
-    of the chip idle.  (Microseconds per row step, measured at 8 iterations
+    of the chip idle, be they a handful (4 images of 1024^2 in 2052 units of 18
+    rows 2.57 ms per 240 iterations, in 936 of 40 2.07).  (Microseconds per row step, measured at 8 iterations
     per launch on 32 and 128 images of 1024^2 with 48 to 256 rows: within 10%
     of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)
     Where every unit has a SIMD of its own the shortest units win, down to
@@ -164,7 +165,6 @@ def wide_rows(H, strips, k, simds):
     n = units.sum(axis=1)
     steps = (units * (-(-H // chunks) + 2 * k)).sum(axis=1) / n  # of a unit, on average
     rounds, rest = np.divmod(n / simds, 2.0)
-    rest = np.where((rounds > 0) & (rest < 0.01), 0.0, rest)  # a handful of units beside the full rounds
     cost = steps * (1.54 * rounds + np.where(rest == 0.0, 0.0, np.where(rest <= 1.0, 0.95, 1.54)))
     return int(R[np.argmin(cost), 0])
 

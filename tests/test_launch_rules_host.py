@@ -22,6 +22,17 @@ def test_wide_rows_fill_the_chip(shapes, k):
         assert units >= 512
 
 
+@pytest.mark.parametrize("n,H,W,k", [(4, 1024, 1024, 8), (4, 1024, 1024, 6), (1, 2048, 2048, 6), (2, 2048, 2048, 6),
+                                     (12, 1024, 1024, 8)])
+def test_wide_rows_leave_no_handful_over(n, H, W, k):
+    """A few units beside two full ones per SIMD start when the others end and
+    take as long again: not one to a hundredth of the SIMDs over."""
+    h, w = np.full(n, H), np.full(n, W)
+    strips = tv._wide_strips(w, tv.WIDE_COLS - 2 * k)
+    units = int(np.sum(strips * -(-h // tv.wide_rows(h, strips, k, 1024))))
+    assert not 2048 < units < 2048 + 11
+
+
 def test_kernel_choice_does_not_walk_the_batch():
     """The choice is made several times per block: its cost must not grow with
     the number of instances."""
