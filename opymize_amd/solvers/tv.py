@@ -138,9 +138,8 @@ CAPTURE_BELOW = 4
 # rows per thread that the tile kernel of several iterations per launch is built for
 MULTI_ROWS = (2, 4, 6, 8)
 
-# rows per unit that the two-column kernel may take (wide_rows)
-WIDE_ROWS = (1, 2, 3, 4, 5, 6, 8, 10, 12, 14, 16, 18, 20, 22, 24, 28, 32, 36, 40, 44, 48, 52, 57, 64, 69, 74, 80, 86, 94, 103, 114, 128,
-             147, 171, 205, 256, 342, 512)
+# rows per unit that the two-column kernel may take (wide_rows): all up to 24, then in steps of 8%
+WIDE_ROWS = tuple(range(1, 25)) + tuple(round(24 * 1.08 ** i) for i in range(1, 41))
 
 
 def wide_rows(H, strips, k, simds):
@@ -155,15 +154,18 @@ def wide_rows(H, strips, k, simds):
     rows 2.57 ms per 240 iterations, in 936 of 40 2.07).  (Microseconds per row step, measured at 8 iterations
     per launch on 32 and 128 images of 1024^2 with 48 to 256 rows: within 10%
     of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)
-    Where every unit has a SIMD of its own the shortest units win, down to
+    Steps of 8% reach every number of chunks up to 13 of any height.  Where
+    every unit has a SIMD of its own the shortest units win, down to
     one row each (960 iterations of one 64^2 image: 8 rows 3.73 ms, 4 rows
     3.34, 1 row 3.01; of one 512^2 image 3.79, 3.38 and, past a unit per SIMD,
     5.65)."""
-    R = np.asarray(WIDE_ROWS)[:, None]
-    chunks = -(-H // R)
+    H, of = np.unique(H, return_inverse=True)
+    strips = np.bincount(of, weights=strips)  # by height
+    R = np.asarray(WIDE_ROWS, dtype=np.float64)[:, None]
+    chunks = np.ceil(H / R)
     units = strips * chunks
     n = units.sum(axis=1)
-    steps = (units * (-(-H // chunks) + 2 * k)).sum(axis=1) / n  # of a unit, on average
+    steps = (units * np.ceil(H / chunks)).sum(axis=1) / n + 2 * k  # of a unit, on average
     rounds, rest = np.divmod(n / simds, 2.0)
     cost = steps * (1.54 * rounds + np.where(rest == 0.0, 0.0, np.where(rest <= 1.0, 0.95, 1.54)))
     return int(R[np.argmin(cost), 0])
