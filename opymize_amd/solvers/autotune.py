@@ -94,6 +94,8 @@ def tune(batch, steps="adaptive", step_bound=0.124, iters=24, widths=None, rpts=
             for rpt in cand:
                 batch.set_multi(m)
                 batch.set_tile(tw, rpt)
+                if m > 1 and rpt != cand[-1] and steps != "adaptive" and batch._use_wide(batch._cfg(steps)):
+                    continue  # a kernel without tiles: timed once, with the tallest for the checks
                 batch.set_start(x0, y0)
                 n = max(m, iters - iters % m)
                 try:

@@ -313,6 +313,7 @@ class TVBatch(object):
         self._strips = np.array([_stream_strips(W, sw) for (H, W) in self.shapes], dtype=np.int64)
         self._units = self._strips * -(-self._H // rows)
         self.total_units = int(self._units.sum())
+        self._wide_now = self._few_units(self.total_units)
         if self._grid_override is None:
             self.sgrid = self._stream_grid(self.total_units)
         else:
@@ -388,6 +389,9 @@ class TVBatch(object):
         2, - / 13.8 / 13.2 with 4; 16 of 1024^2 (2300) 13.5 / - / 14.4 with 2, 11.3 /
         - / 10.6 with 3; 6 of 1024^2 (860) 6.1 / - / 5.1 with 2."""
         return self._wide_fits(cfg) and self._wide_now
+
+    def _few_units(self, units):
+        return units < WIDE_UNITS.get(self.multi, units + 1)
 
     def _wide_fits(self, cfg):
         return (self.multi_kernel == "auto" and self.multi > 1 and self.C == 1 and self.dtype == torch.float32
@@ -475,7 +479,7 @@ class TVBatch(object):
             if self._grid_override is None:
                 self.sgrid = self._stream_grid(units)
             self._stream_now = units >= self.stream_min_units
-            self._wide_now = units < WIDE_UNITS.get(self.multi, units + 1)
+            self._wide_now = self._few_units(units)
             if self._size_wide(running):
                 self._stream_units()
         return nrun

@@ -253,6 +253,24 @@ def test_autotune_considers_iterations_per_launch(gpu):
     autotune._cache.clear()
 
 
+def test_autotune_times_a_kernel_without_tiles_once(gpu):
+    """One-channel FP32: the two-column kernel takes no tile, so one candidate
+    per number of iterations per launch; tiles where the batch's size gives it
+    to them (2 per launch from 2048 units)."""
+    from opymize_amd.solvers import autotune
+    from opymize_amd.solvers.tv import TVBatch
+    for n, side, per in ((3, 70, {2: 1, 3: 1}), (600, 130, {2: 4, 3: 1})):
+        bat = TVBatch([rects(side, side, 3)] * n, 4.0, "l2", precision="float")
+        shapes = set()
+        solve = bat.solve
+        bat.solve = lambda **kw: (shapes.add((bat.multi, bat.rpt)), solve(**kw))[1]
+        autotune._cache.clear()
+        best = autotune.tune(bat, steps="accel", iters=12, blocks=(12,), multis=(1, 2, 3))
+        autotune._cache.clear()
+        assert {m: sum(s[0] == m for s in shapes) for m in per} == per, (n, shapes)
+        assert best["multi"] in (1, 2, 3)
+
+
 @pytest.mark.parametrize("multi,rpt", [(1, 8), (4, 4)])
 def test_launch_shapes_give_the_same_iterates(gpu, multi, rpt):
     """One block per running tile (the default), the persistent grid of
