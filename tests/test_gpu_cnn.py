@@ -365,3 +365,30 @@ def test_partial_sums_over_segments(gpu, nb):
     assert bool(((a.double() - p.sum(0)).abs() <= tol).all())
     w = a[:9 * 1024].view(9, 32, 32).transpose(1, 2).reshape(-1)
     assert torch.equal(b[:9 * 1024], w) and torch.equal(b[9 * 1024:], a[9 * 1024:])
+
+
+def test_layer_entry_points_equal_the_fused_ones(gpu):
+    """opy_conv3x3_prep_weights of each layer and direction against
+    opy_conv3x3_prep_all, and opy_conv3x3_fwd_bf16 with opy_relu_bwd_f32 against
+    opy_conv3x3_bwd_data: the same bits."""
+    from opymize_amd.warmstart.cnn import ConvNet, _call
+    from opymize_amd import _hip
+    rng = np.random.default_rng(12)
+    net = ConvNet(layers=3, n_in=32, n_out=32, seed=8)
+    net._prep()
+    s = _hip.stream()
+    for l in range(3):
+        for flip, ref in ((0, net._wf[l]), (1, net._wb[l])):
+            out = torch.zeros_like(ref)
+            _call("opy_conv3x3_prep_weights", _hip.ptr(net.W(l)), _hip.ptr(out), flip, s)
+            assert torch.equal(out.view(torch.int16), ref.view(torch.int16))
+    N, H, W = 2, 19, 45
+    g, mask = (torch.as_tensor(rng.standard_normal((N, H, W, 32)).astype(np.float32)).cuda() for _ in range(2))
+    mask[0, 3] = 0.0
+    a, b = torch.full_like(g, 7.0), torch.full_like(g, 7.0)
+    _call("opy_conv3x3_bwd_data", _hip.ptr(g), _hip.ptr(a), _hip.ptr(net._wb[1]), _hip.ptr(mask), N, H, W, net.grid, s)
+    _call("opy_conv3x3_fwd_bf16", _hip.ptr(g), _hip.ptr(b), _hip.ptr(net._wb[1]), None, N, H, W, 0, net.grid, s)
+    raw = b.clone()
+    _call("opy_relu_bwd_f32", _hip.ptr(b), _hip.ptr(mask), b.numel(), s)
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    assert torch.equal(b, torch.where(mask > 0, raw, torch.zeros_like(raw)))

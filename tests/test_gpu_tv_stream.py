@@ -160,14 +160,17 @@ def test_stream_matches_oracle_and_certifies(gpu):
     assert [r["gap"] for r in res["stream"]] == [r["gap"] for r in res["tile"]]
 
 
-def test_auto_switches_to_tiles_when_few_units_run(gpu):
+@pytest.mark.parametrize("precision,C", [("double", 1), ("float", 2)])
+def test_auto_switches_to_tiles_when_few_units_run(gpu, precision, C):
     """multi_kernel="auto" streams while enough units run and takes the tile
     kernel once instances drop out (here: as soon as one has certified); the
     whole solve certifies with the iterations, gaps and iterates of a solve on
-    the tile kernel alone."""
+    the tile kernel alone.  (One-channel FP32 batches have a kernel of their own,
+    see test_gpu_tv_wide.py.)"""
     out = {}
     for kernel in ("auto", "tile"):
-        bat, *_ = _batch("float", 4, kernel, seed=3, data="l2", rows=16)
+        bat, *_ = _batch(precision, 4, kernel, seed=3, data="l2", rows=16, C=C)
+        assert not bat._use_wide(bat._cfg("accel"))
         if kernel == "auto":
             bat.stream_min_units = bat.total_units  # stream only while every instance runs
             bat.solve(steps="accel", step_bound=0.124, max_iters=40, block_iters=40, tol=1e-30)

@@ -94,6 +94,37 @@ def test_wide_launch_shapes(gpu, multi):
         assert out[None][1] == out[g][1]
 
 
+@pytest.mark.parametrize("multi,block,graph", [(8, 130, False), (7, 130, False), (6, 64, False), (5, 68, False),
+                                               (3, 130, True), (3, 130, False), (8, 72, False)])
+def test_blocks_longer_than_a_step_table(gpu, multi, block, graph):
+    """One table holds the steps of at most 64 iterations, in whole launches
+    (63 for 7 or 3 per launch, 60 for 5): blocks that take a second and a third
+    one carry the schedule on from table to table; the iterates and steps of
+    single launches, bit for bit, and the same over a second solve."""
+    from opymize_amd.solvers import tv
+    imgs = [rects(H, W, 50 + i) for i, (H, W) in enumerate([(40, 129), (97, 1), (64, 150), (9, 300)])]
+    out = []
+    for m, g in ((multi, graph), (1, True)):
+        bat = tv.TVBatch(imgs, [2.0, 9.0, 15.0, 19.0], ["l2", "l1", "l2", "l2"], multi=m)
+        names = []
+        call = bat._call
+        bat._call = lambda name, *a: (names.append(name), call(name, *a))[1]
+        for _ in range(2):
+            bat.set_start(None, None)
+            res = bat.solve(steps="accel", step_bound=0.124, step_factor=4.0, max_iters=3 * block, block_iters=block,
+                            tol=1e-30, use_graph=g)
+        out.append((bat.solution(), [r["gap"] for r in res], bat.steps_state()))
+        if m > 1 and not g:
+            per = tv.WIDE_TABLE - tv.WIDE_TABLE % m
+            assert names.count("opy_tv_wide_steps") == 6 * -(-(block - block % m) // per)
+            assert names.count("opy_tv_wide_f32") == 6 * (block // m)
+    for a, b in zip(out[0][0][0] + out[0][0][1], out[1][0][0] + out[1][0][1]):
+        np.testing.assert_array_equal(a, b)
+    assert out[0][1] == out[1][1]
+    for a, b in zip(out[0][2], out[1][2]):
+        assert (a["tau"], a["sigma"]) == (b["tau"], b["sigma"])
+
+
 def test_kernel_may_change_between_blocks(gpu, monkeypatch):
     """Fewer than 6 iterations per launch: one column per lane while the batch
     is large, two from the check on at which enough instances stopped; captured
@@ -151,6 +182,27 @@ def test_wide_units_follow_the_running_instances(gpu):
                               (bat.unit_off, bat._strips, bat.stream_rows)):
         counts = (strips * -(-bat._H // rows))[active]
         np.testing.assert_array_equal(off.cpu().numpy()[:nrun + 1], np.concatenate([[0], np.cumsum(counts)]))
+
+
+def test_units_entry_points_agree(gpu):
+    """opy_tv_stream_units writes the prefix that opy_tv_wide_units writes
+    beside its own, for every number of iterations per launch."""
+    import torch
+    from opymize_amd import _hip
+    from opymize_amd.solvers import tv
+    P = _hip.ptr
+    bat = tv.TVBatch([rects(H, W, 9 + i) for i, (H, W) in enumerate(SHAPES)], 3.0, "l2", multi=8)
+    bat.solve(steps="accel", step_bound=0.124, max_iters=8, block_iters=8, tol=1e-30)
+    for k in range(2, 9):
+        for rows in (1, 16, 128):
+            a, b, c = (torch.full((bat.B + 1,), -1, dtype=torch.int32, device="cuda") for _ in range(3))
+            bat._call("opy_tv_stream_units", P(bat.insts), P(bat.active_inst), P(bat.nact), P(a), k, rows,
+                      _hip.stream())
+            bat._call("opy_tv_wide_units", P(bat.insts), P(bat.active_inst), P(bat.nact), k, P(b), rows, P(c), 32,
+                      _hip.stream())
+            counts = [tv._stream_strips(W, 64 - 2 * k) * -(-H // rows) for H, W in SHAPES]
+            np.testing.assert_array_equal(a.cpu().numpy(), np.concatenate([[0], np.cumsum(counts)]))
+            assert torch.equal(a, b)
 
 
 def test_wide_graph_replays_equal_eager(gpu, monkeypatch):
