@@ -1,10 +1,11 @@
 """Batched fused PDHG for the multi-label lifting model.
 
 Many instances of opymize_amd.lifting.sublabel_tv -- images of uneven size
-and uneven label count -- iterate together: two kernel launches per
-iteration over the tiles of the still-running instances (csrc/lift.hip),
-blocks of iterations captured in HIP graphs, an FP64 gap per instance on the
-device every check, and a device-side list of the running instances.  The
+and uneven label count -- iterate together: one kernel launch per iteration
+over the tiles of the still-running instances, or two (csrc/lift.hip,
+_one_pass_serves), blocks of short iterations captured in HIP graphs, an FP64
+gap per instance on the device every check, and a device-side list of the
+running instances.  The
 iterates equal those of PDHG(G, F, A).solve(steps="precond") of each
 instance's model (reference pdhg.py:229-315 with its steps "precond",
 pdhg.py:189-200, made constant on the coupled blocks), up to rounding.
@@ -155,8 +156,10 @@ class LiftBatch(object):
     @staticmethod
     def _room_for(nbytes):
         """Whether nbytes can be taken and as much again stays free."""
-        cached = torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
-        return 2 * nbytes <= torch.cuda.mem_get_info()[0] + cached
+        free = torch.cuda.mem_get_info()[0]
+        if 2 * nbytes <= free:  # 6 us; the allocator's own counts take 70 each
+            return True
+        return 2 * nbytes <= free + torch.cuda.memory_reserved() - torch.cuda.memory_allocated()
 
     # -- kernels ---------------------------------------------------------------
     def _sfx(self):
@@ -290,7 +293,9 @@ class LiftBatch(object):
         """Iterate from the current state (zeros after construction or reset())
         until every instance has |relgap| < tol and both infeasibilities
         < tol_infeas, or max_iters; the test runs every
-        block_iters*check_every iterations.  Returns self.results()."""
+        block_iters*check_every iterations.  use_graph=True captures blocks in
+        graphs where that is the faster form (_captured).  Returns
+        self.results()."""
         if block_iters < 1 or check_every < 1:
             raise ValueError("block_iters and check_every must be positive")
         tol_infeas = tol if tol_infeas is None else tol_infeas
