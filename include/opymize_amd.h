@@ -540,7 +540,7 @@ int opy_lift_dual_f64(const double* Ub, const double* rb, double* p, double* z, 
                       const opy_lift_inst_t* insts, const int32_t* active_inst, const int32_t* act_off,
                       const int32_t* nact, int kmax, int grid, void* stream);
 /* both passes in one: reads U, r, p, z and f, writes r in place and U, p, z to their other buffers; the iterates of
- * a primal and a dual pass.  kmax <= 32 (FP64: 16). */
+ * a primal and a dual pass up to rounding.  kmax <= 32 (FP64: 16). */
 int opy_lift_iter_f32(const float* U_in, float* U_out, float* r, const float* p_in, float* p_out, const float* z_in,
                       float* z_out, const float* f, const opy_lift_inst_t* insts, const int32_t* active_inst,
                       const int32_t* act_off, const int32_t* nact, int kmax, int grid, void* stream);

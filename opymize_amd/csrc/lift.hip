@@ -293,14 +293,18 @@ __global__ void __launch_bounds__(256) lift_dual_kernel(const T* __restrict__ Ub
 // the tile: reads U, r, p, z and f, writes U, r, p, z, 12 planes instead of the
 // two passes' 20 (x_bar of both never leaves the chip).  Neighbouring tiles read
 // U, p and nu of the last iteration, so those go from one set of buffers to the
-// other; r stays in place.  4 x 512^2, L = 16, FP32: 264 us for the two passes
-// (4.8 TB/s), 214 us here (3.5 TB/s of the 12 planes): the bytes fell by 40%, and
-// what bounds it now is the latency of a tile's four phases (halo, primal loads,
-// simplex, dual loads), with the 4 blocks per CU that LDS and registers allow.
+// other; r stays in place.  4 x 512^2, L = 16, FP32: 264 us for the two passes,
+// 213 us here.  HBM bounds it: the second half's p and z and the halo row (a
+// quarter of a tile's U, p and nu) come from memory again, 775 MB read where 382
+// would do, and with the 377 MB written that is 5.4 TB/s, nine tenths of what a
+// copy reaches (VALU busy 35%, 13 wavefronts per CU).
 //
-// The second half reads p and z again, through the caches, and takes r_bar from
-// LDS: its loop over the pieces is then a loop in the code as well, and the
-// registers hold one half's values at a time.
+// The second half reads p and z again and takes r_bar from LDS: its loop over
+// the pieces is then a loop in the code as well, and the registers hold one
+// half's values at a time (kept in registers instead, p and z took 206 us, not
+// worth the code).  The FP32 ball projection scales by v_rsq_f32 (within 1 ulp)
+// where the dual pass divides by a square root, so the two forms' p differ in
+// the last place.
 constexpr int kIChunk = 4;  // pieces whose loads go out together
 
 template <typename T, int KMAX>

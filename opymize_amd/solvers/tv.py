@@ -3,14 +3,15 @@
 One engine serves both the drop-in single-instance path (PDHG.solve on a
 recognised TV-L2/TV-L1 model) and the batched solver over many instances of
 uneven size.  Per iteration it launches one fused pass (two with passes=2)
-and, with adaptive steps, one small per-instance rule kernel; every
-`block_iters` iterations it evaluates the FP64 primal-dual gap, marks
-converged instances and compacts
-the list of running instances -- all on the device, so a whole block is one
-hipGraph replay and the host only reads the number of running instances and
-their tiles, which sizes the next launches (one block per running tile: the
-hardware dispatcher then keeps the tiles in flight contiguous in memory,
-which streams faster than a persistent grid whose blocks drift apart).
+and, with adaptive steps, one small per-instance rule kernel; with the other
+rules it can run several iterations per launch.  Every `block_iters`
+iterations it evaluates the FP64 primal-dual gap, marks converged instances
+and compacts the list of running instances -- all on the device, so a block
+is one hipGraph replay (blocks of few long launches are issued plainly, see
+_captured) and the host only reads the list of running instances, which
+sizes the next launches (one block per running tile: the hardware dispatcher
+then keeps the tiles in flight contiguous in memory, which streams faster
+than a persistent grid whose blocks drift apart).
 
 Model of instance b: min_x G_b(x) + tvw_b * sum_p |grad x(p)|_F with
 G_b = 0.5*lam_b*|x - f_b|^2 (data="l2") or lam_b*|x - f_b|_1 (data="l1"),
@@ -203,7 +204,10 @@ class TVBatch(object):
             (decided at each check), else take tiles with min(K, 4) iterations
             per launch; preconditioned steps take tiles.  Every choice gives
             the iterates of single launches bit for bit
-    stream_rows: rows per unit of the streaming kernel
+    stream_rows: rows per unit of the one-column streaming kernel
+            ("stream", and "auto" where it takes that kernel)
+    grid:   blocks per launch: None one per running tile or unit, 0 as many
+            as are resident at once, n that many
     """
 
     def __init__(self, images, lam, data="l2", tvw=1.0, precision="float", tile=(64, 4), h=(1.0, 1.0),
@@ -775,6 +779,9 @@ class TVBatch(object):
         """Iterate until every instance is certified (|relgap| < tol and
         infeasibility < tol_infeas) or max_iters; the test runs every
         block_iters*check_every iterations.  Returns self.results().
+
+        use_graph=True captures blocks and checks in graphs where that is the
+        faster form (_captured); False issues every launch plainly.
 
         fallback=True (for warm starts): the gap of the start point is
         recorded, and an instance whose gap has not improved at the first
