@@ -652,6 +652,9 @@ def main():
     bcfg = bat._cfg(args.step_rule)
     kind = "wide" if bat._use_wide(bcfg) else "stream" if bat.multi > 1 and bat._use_stream(bcfg) else "multi"
     unit_rows = {"wide": bat.wrows, "stream": bat.stream_rows}.get(kind)
+    if kind == "wide":  # an image's rows are shared evenly
+        H = max(h for h, w in bat.shapes)
+        unit_rows = -(-H // -(-H // unit_rows))
     lane_cols = 128 if kind == "wide" else 64
     variant = "adaptive" if args.step_rule == "adaptive" else "accelerated steps"
     k_launch = 1

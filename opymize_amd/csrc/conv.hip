@@ -296,7 +296,7 @@ void launch_conv(const TX* x, TY* y, const void* wt, const float* bias, const fl
 // by byte alignment, and an input row serves the three output rows it borders,
 // so a row costs 3 LDS reads for 9 matrix instructions.  32 x 128^2: 107 -> 35 us
 // a layer, 4.3 TB/s of x, g and the partials; the matrix cores are busy for 13% of
-// it, the LDS for 40% (most of it bank conflicts of the channel-major stores).
+// it, the LDS for 40% (70% of that bank conflicts).
 constexpr int kGW = 32, kGH = 8;          // tile
 constexpr int kGP = 40;                   // bf16 elements per (row, channel) in LDS, 34 / 32 used
 __global__ void __launch_bounds__(256) conv3x3_wgrad_kernel(const float* __restrict__ x, const float* __restrict__ g,

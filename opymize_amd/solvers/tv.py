@@ -152,14 +152,15 @@ def wide_rows(H, strips, k, simds):
     SIMD runs two units at once, in 1.54 of the time units that one alone
     takes 0.95 of, and those left over when the others have ended leave most
     of the chip idle, be they a handful (4 images of 1024^2 in 2052 units of 18
-    rows 2.57 ms per 240 iterations, in 936 of 40 2.07).  (Microseconds per row step, measured at 8 iterations
-    per launch on 32 and 128 images of 1024^2 with 48 to 256 rows: within 10%
-    of the launch times throughout, e.g. 147 rows 251 us, 128 rows 321 us.)
-    Steps of 8% reach every number of chunks up to 13 of any height.  Where
-    every unit has a SIMD of its own the shortest units win, down to
-    one row each (960 iterations of one 64^2 image: 8 rows 3.73 ms, 4 rows
-    3.34, 1 row 3.01; of one 512^2 image 3.79, 3.38 and, past a unit per SIMD,
-    5.65)."""
+    rows 2.57 ms per 240 iterations, in 936 of 40 2.07).  (Microseconds per row
+    step, measured at 8 iterations per launch on 32 and 128 images of 1024^2
+    with 48 to 256 rows: within 10% of the launch times throughout, e.g. 147
+    rows 251 us, 128 rows 321 us.  With 2 to 5 per launch the rows chosen come
+    within 8% of the best of 16, 32, 64, 128 and 256.)  Steps of 8% reach every
+    number of chunks up to 13 of any height.  Where every unit has a SIMD of
+    its own the shortest units win, down to one row each (960 iterations of one
+    64^2 image: 8 rows 3.73 ms, 4 rows 3.34, 1 row 3.01; of one 512^2 image
+    3.79, 3.38 and, past a unit per SIMD, 5.65)."""
     H, of = np.unique(H, return_inverse=True)
     strips = np.bincount(of, weights=strips)  # by height
     R = np.asarray(WIDE_ROWS, dtype=np.float64)[:, None]
