@@ -167,7 +167,7 @@ def wide_rows(H, strips, k, simds):
     chunks = np.ceil(H / R)
     units = strips * chunks
     n = units.sum(axis=1)
-    steps = (units * np.ceil(H / chunks)).sum(axis=1) / n + 2 * k  # of a unit, on average
+    steps = (units * np.ceil(H / np.maximum(chunks, 1.0))).sum(axis=1) / n + 2 * k  # of a unit, on average
     rounds, rest = np.divmod(n / simds, 2.0)
     cost = steps * (1.54 * rounds + np.where(rest == 0.0, 0.0, np.where(rest <= 1.0, 0.95, 1.54)))
     return int(R[np.argmin(cost), 0])
@@ -341,7 +341,7 @@ class TVBatch(object):
         if self.C != 1 or self.dtype != torch.float32:
             return False
         work = self._wide_work
-        share = -(-16 * int(work[running].sum()) // int(work.sum())) if len(running) else 0
+        share = -(-16 * int(work[running].sum()) // max(1, int(work.sum()))) if len(running) else 0
         if share == self._wide_sized or share == 0:
             return False
         self._wide_sized = share

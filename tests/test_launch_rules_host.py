@@ -22,6 +22,12 @@ def test_wide_rows_fill_the_chip(shapes, k):
         assert units >= 512
 
 
+def test_wide_rows_pass_over_empty_images():
+    H, W = np.array([0, 700, 300, 0]), np.array([5, 900, 400, 0])
+    strips = tv._wide_strips(W, 112)
+    assert tv.wide_rows(H, strips, 8, 1024) == tv.wide_rows(H[1:3], strips[1:3], 8, 1024)
+
+
 @pytest.mark.parametrize("n,H,W,k", [(4, 1024, 1024, 8), (4, 1024, 1024, 6), (1, 2048, 2048, 6), (2, 2048, 2048, 6),
                                      (12, 1024, 1024, 8)])
 def test_wide_rows_leave_no_handful_over(n, H, W, k):
