@@ -62,8 +62,9 @@ def test_gradient_divergence(gpu, dtype, dims, C, scheme):
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("C,offset", [(1, 1), (1, 0), (4, 0), (2, 3)])
-def test_gradient_divergence_2d_views(gpu, dtype, C, offset):
-    """The 2-D forward kernels on views at element offsets (the 2-vector
+@pytest.mark.parametrize("scheme", ["forward", "centered"])
+def test_gradient_divergence_2d_views(gpu, dtype, C, offset, scheme):
+    """The 2-D kernels of both schemes on views at element offsets (the 2-vector
     accesses of C = 1 need an aligned field, else the scalar form runs), for
     C = 1, 2 and 4, with and without add, against the oracle matrices."""
     from opymize_amd.linear import GradientOp
@@ -72,8 +73,8 @@ def test_gradient_divergence_2d_views(gpu, dtype, C, offset):
     dims = (37, 45)
     h = rng.uniform(0.5, 2, 2)
     w = rng.uniform(0.5, 2, C)
-    op = GradientOp(dims, C, scheme="forward", imageh=h, weights=w)
-    G = ops.grad_matrix(dims, C, h, w, "forward")
+    op = GradientOp(dims, C, scheme=scheme, imageh=h, weights=w)
+    G = ops.grad_matrix(dims, C, h, w, scheme)
     x = rng.standard_normal(op.x.size)
     p = rng.standard_normal(op.y.size)
     xr = x.astype(dtype).astype(np.float64)
