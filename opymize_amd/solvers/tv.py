@@ -267,8 +267,9 @@ class TVBatch(object):
         # units (about four wavefronts per SIMD), else takes the tile kernel
         self.stream_min_units = STREAM_MIN_UNITS
         self._stream_now = self._wide_now = True
-        self.set_multi(multi)
+        self.multi = 1  # until stream_rows is set: one layout, not two
         self.set_stream_rows(stream_rows)
+        self.set_multi(multi)
         self.set_tile(*tile)
         self.graph = None
         self.cur = 0  # buffer holding the current iterate of the running instances
